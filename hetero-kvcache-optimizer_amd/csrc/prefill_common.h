@@ -1,11 +1,26 @@
-// Shared by the two chunked-prefill kernels (prefill_zones.hip: fp16 zone tiles and
-// the causal chunk; prefill_attn.hip: INT4 tiles and the entry point).
+// Shared by the chunked-prefill sources (prefill_attn.hip: entry point, attention kernel,
+// combine kernel; prefill_stage.h: the staging policies; prefill_flat.h: the tile loop).
 //
-// A launch with both kinds of keys runs the zone kernel first.  It leaves, per
-// (sequence, query head, query row), the online-softmax state of the zone and chunk
-// tokens in a workspace -- the unnormalized output O (relative to the running max m),
-// m, and the running sums of the two lane halves -- and the INT4 kernel starts from that
-// state, so the result is the softmax over all keys as from one pass.
+// Rows.  The n_rep query heads of a GQA group share their kv head's keys, so a (sequence,
+// kv head) pair is one attention problem of Sq x n_rep rows; row r is query r / n_rep of
+// head r % n_rep.  A unit is kUnitRows consecutive rows, whatever n_rep: no wave sits on
+// an absent head (with one wave per head, n_rep = 1 left three of four waves idle and
+// n_rep = 7 one of eight: 512 queries of 32 heads over 4096 keys each, 158 -> 90 us with
+// the repacking of the keys; 2048 queries of 28/4 heads over 4160 keys and themselves, 239
+// -> 204 us).
+//
+// Work.  A unit's keys are tiles of 64 tokens of two kinds, each with its own staging: fp16
+// (the zones' tiles, then the chunk's up to the unit's last query) and INT4.  A piece is
+// 1 / pieces of a unit's tiles of one kind, one workgroup's work.  It leaves its
+// online-softmax state (O relative to the row max m, m, and the row sum l, in float32) in
+// its state rows, unless it is all of the unit's keys: then it writes the output.
+//   kFinishOut      one kind, one piece per unit: every workgroup writes its unit's output
+//   kFinishPieces   all pieces of all units, of both kinds, in one grid; the combine kernel
+//                   merges their states
+//   kFinishSerial   both kinds, one piece each: the fp16 kernel runs first, the INT4 kernel
+//                   merges its states into its own and writes the output
+// A workgroup takes one piece: with a loop over several, the tile loop's register
+// allocation (248 of 256) no longer holds.
 #pragma once
 
 #include "hkv_internal.h"
@@ -21,18 +36,12 @@ typedef uint32_t pu2 __attribute__((ext_vector_type(2)));
 constexpr int kPfQ = 32;             // query rows per wave
 constexpr int kPfT = 64;             // tokens per tile
 constexpr float kPfLog2e = 1.4426950408889634f;
-constexpr int kStateFloats = 132;    // O[128], m, l (lanes 0-31), l (lanes 32-63), pad
+constexpr int kUnitRows = 256;       // rows per unit: 8 waves of kPfQ
+constexpr int kStateFloats = 132;    // a row's state: O[128], m, l, pad
+enum : int { kKindF16 = 0, kKindInt4 = 1 };
 
-struct PfZone {
-    const uint16_t* k;
-    const uint16_t* v;
-    int cap;
-    int max_len;
-    const int32_t* lens;
-};
-
-// Where the zone kernel reads the fp16 tiles of one source (a zone, or the causal chunk
-// in the zone layout): K rows [B*Hkv][cap][128], V tiles [B*Hkv][cap/16][16 x 128].
+// Where the fp16 tiles of one source lie (a zone, or the causal chunk in
+// the zone layout): K rows [B*Hkv][cap][128], V tiles [B*Hkv][cap/16][16 x 128].
 struct PfSrc {
     const uint16_t* k;
     const uint16_t* v;
@@ -40,14 +49,20 @@ struct PfSrc {
     int pad;
 };
 
+enum : int { kFinishOut = 0, kFinishPieces = 1, kFinishSerial = 2 };
+
 struct PrefillParams {
     int B, Hkv, nrep, Sq;
     float scale_log2;
-    int q_bf16, c_bf16, out_bf16;   // q / chunk / out dtype is bfloat16 (else fp16)
+    int q_bf16, out_bf16;           // q / out dtype is bfloat16 (else fp16)
     const uint16_t* q;
     int64_t q_sb, q_sh, q_st;
-    int nz;
-    PfZone z[HKV_MAX_F16_ZONES];
+    int has_chunk;
+    int zone_max[HKV_MAX_F16_ZONES];
+    const int32_t* zone_lens[HKV_MAX_F16_ZONES];
+    // the fp16 sources in tile order: zones 0..2 (unused ones empty), then the chunk;
+    // indexed at run time, so that no source's pointers stay in registers
+    PfSrc src[HKV_MAX_F16_ZONES + 1];
     const uint8_t* pool;
     uint32_t pool_blocks;        // record counts capped at 2^31 (block ids are int32), so the
     const uint8_t* staging;      // range check is a 32-bit scalar compare; staging records are
@@ -57,20 +72,20 @@ struct PrefillParams {
     int bt_stride;
     const int32_t* int4_lens;
     int int4_max_len;
-    const uint16_t* ck;          // causal chunk K/V [B][Hkv][Sq][128] (may be null)
-    const uint16_t* cv;
-    int64_t c_sb, c_sh, c_st;
     uint16_t* out;
     int64_t o_sb, o_sh, o_st;
     int* err;
-    float* state;                // [B][Hq][Sq][kStateFloats] zone-kernel state (may be null)
-    const uint16_t* czk;         // the causal chunk in the zone layout: K rows [B*Hkv][ccap][128]
-    const uint16_t* czv;         // and V tiles [B*Hkv][ccap/16][16 x 128] (null without a chunk)
-    int ccap;
-    // the zone kernel's sources in tile order: zones 0..2 (unused ones empty), then the
-    // chunk; indexed at run time, so that no source's pointers stay in registers
-    PfSrc src[HKV_MAX_F16_ZONES + 1];
+    int units;                   // units per (sequence, kv head)
+    int finish;                  // kFinish*
+    int pieces[2];               // per unit, by kind (0: the launch has no tiles of the kind)
+    float* state;                // state rows [.][kStateFloats]
 };
+
+// First state row of piece s of kind `kind` of unit `unit` (counted over all pairs).
+__device__ __forceinline__ int64_t piece_row(const PrefillParams& p, int kind, int unit, int s) {
+    const int per_unit = p.pieces[0] + p.pieces[1];
+    return ((int64_t)unit * per_unit + (kind == kKindInt4 ? s : p.pieces[kKindInt4] + s)) * kUnitRows;
+}
 
 // Tile counts of one sequence: INT4 tiles, each zone's tiles, and the causal chunk's
 // tiles up to query row q_end (exclusive).
@@ -81,20 +96,14 @@ struct TileMap {
 };
 
 __device__ __forceinline__ void make_tile_map(const PrefillParams& p, int b, int q_end, TileMap& tm) {
-    tm.len4 = p.int4_lens ? min(max(p.int4_lens[b], 0), p.int4_max_len) : p.int4_max_len;
+    tm.len4 = p.int4_lens ? min(max(load_uniform_i32(p.int4_lens, b), 0), p.int4_max_len) : p.int4_max_len;
     tm.n4 = (tm.len4 + kPfT - 1) / kPfT;
 #pragma unroll
     for (int zi = 0; zi < HKV_MAX_F16_ZONES; ++zi) {
-        tm.lenz[zi] = 0;
-        if (zi < p.nz) tm.lenz[zi] = p.z[zi].lens ? min(max(p.z[zi].lens[b], 0), p.z[zi].max_len) : p.z[zi].max_len;
+        tm.lenz[zi] = p.zone_lens[zi] ? min(max(load_uniform_i32(p.zone_lens[zi], b), 0), p.zone_max[zi]) : p.zone_max[zi];
         tm.nz_t[zi] = (tm.lenz[zi] + kPfT - 1) / kPfT;
     }
-    tm.nc = p.ck ? (min(q_end, p.Sq) + kPfT - 1) / kPfT : 0;
-}
-
-// The state of query row `qrow` of query head `qh` of sequence b.
-__device__ __forceinline__ float* state_row(const PrefillParams& p, int b, int qh, int qrow) {
-    return p.state + (((int64_t)b * p.Hkv * p.nrep + qh) * p.Sq + qrow) * kStateFloats;
+    tm.nc = p.has_chunk ? (min(q_end, p.Sq) + kPfT - 1) / kPfT : 0;
 }
 
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
@@ -119,8 +128,14 @@ __device__ __forceinline__ pu4 bf16x8_to_f16(pu4 w, bool& over) {
     return r;
 }
 
+// Four output dims at `op`: x times inv, rounded to the output dtype.
+__device__ __forceinline__ void store_out4(const PrefillParams& p, uint16_t* op, pf4 x, float inv) {
+    *(pu2*)op = p.out_bf16 ? pu2{pack2bf(x[0] * inv, x[1] * inv), pack2bf(x[2] * inv, x[3] * inv)}
+                           : pu2{pack2(x[0] * inv, x[1] * inv), pack2(x[2] * inv, x[3] * inv)};
+}
+
 // Writes this lane's final output: acc[db][4j + i] is O^T[dim 32db + 8j + 4hh + i][its
-// query row], l the row's softmax sum.
+// row], l the row's softmax sum.
 __device__ __forceinline__ void write_out(const PrefillParams& p, int b, int qh, int qrow, int hh,
                                           const pf16v (&acc)[4], float l) {
     const float inv = l > 0.f ? 1.0f / l : 0.f;
@@ -128,18 +143,9 @@ __device__ __forceinline__ void write_out(const PrefillParams& p, int b, int qh,
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int d = 32 * db + 8 * j + 4 * hh;
-            if (p.out_bf16)
-                *(pu2*)(op + d) = pu2{pack2bf(acc[db][4 * j + 0] * inv, acc[db][4 * j + 1] * inv),
-                                      pack2bf(acc[db][4 * j + 2] * inv, acc[db][4 * j + 3] * inv)};
-            else
-                *(pu2*)(op + d) = pu2{pack2(acc[db][4 * j + 0] * inv, acc[db][4 * j + 1] * inv),
-                                      pack2(acc[db][4 * j + 2] * inv, acc[db][4 * j + 3] * inv)};
-        }
+        for (int j = 0; j < 4; ++j)
+            store_out4(p, op + 32 * db + 8 * j + 4 * hh,
+                       pf4{acc[db][4 * j + 0], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]}, inv);
 }
-
-// Launches the zone kernel (fp16 zone tiles and the causal chunk) over every sequence.
-int launch_prefill_zones(const PrefillParams& p, int ngrp, hipStream_t stream);
 
 }  // namespace hkv

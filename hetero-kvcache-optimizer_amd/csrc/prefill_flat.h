@@ -1,8 +1,7 @@
-// The tile loop shared by the two chunked-prefill kernels (prefill_attn.hip: INT4
-// tiles; prefill_zones.hip: fp16 zone tiles and the causal chunk).  A workgroup is 8
-// waves over one kv head: wave w takes query head 4 grp + (w & 3) of the GQA group and
-// query rows q0 + 32 (w >> 2) .. +31 (kPfQ rows per wave, 64 per workgroup).  Per
-// 64-token tile t every wave runs, with v_mfma_f32_32x32x16_f16,
+// The tile loop of the chunked-prefill kernel, over any kind of tile (the staging
+// policies are in prefill_stage.h).  A workgroup is 8 waves over one unit of 256 rows of
+// one kv head; wave w takes rows 32 w .. +31.  Per 64-token tile t every wave runs, with
+// v_mfma_f32_32x32x16_f16,
 //   A: S(t+1)^T = K(t+1) . Q^T (16 MFMAs) beside the softmax of S(t) -> P(t)
 //   B: O^T += V(t)^T . P(t)^T (16 MFMAs) beside the staging of tile t+2 (this wave's
 //      16-token quarter of the K rows, waves 0-3, or of the V^T rows, waves 4-7) and
@@ -12,7 +11,8 @@
 // the MFMAs; sched_group_barrier asks the scheduler for that interleave.  Four LDS
 // tile buffers rotate (tile t: V^T and biases read; t+1: K rows read; t+2: written).
 // Tiles past the last one are empty (valid length 0), so every tile does the same work
-// and no MFMA or accumulator update sits behind a branch.
+// and no MFMA or accumulator update sits behind a branch.  (Leaving the unrolled round
+// after the last tile instead costs ~20 registers, which spill.)
 //
 // The S^T accumulator of lane (query n, half hh) holds tokens 8j + 4hh + i of each
 // 32-token block, exactly the 8-token k-slices the P^T operand needs, so P never
@@ -34,7 +34,7 @@ typedef _Float16 fh2 __attribute__((ext_vector_type(2)));
 constexpr int kFlatBufs = 4;
 constexpr int kFlatWaves = 8;
 constexpr int kFlatThreads = kFlatWaves * 64;
-constexpr int kFlatQ = 2 * kPfQ;                     // query rows per workgroup
+static_assert(kFlatWaves * kPfQ == kUnitRows, "one unit per workgroup");
 constexpr int kKRow = kHeadDim * 2 + 16;
 constexpr int kVRow = kPfT * 2 + 16;
 constexpr int kVOff = kPfT * kKRow;
@@ -65,21 +65,11 @@ __device__ __forceinline__ void flat_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// A wave's place: staging share wt (of 4) and lane; its lane's query (row / n_rep) and the
+// wave's lowest one.
 struct FlatWave {
-    int b, h, wt, lane, n, hh, qrow, qb;
+    int b, h, wt, lane, n, hh, qrow, q_lo;
 };
-
-// The workgroup's query block and (kv head, GQA group) index.  Dispatch goes round-robin
-// over the 8 XCDs by linear workgroup id, so with qb = lin / HG and hg = lin % HG (HG =
-// gridDim.y, the head-group count) every workgroup of one head group runs on the same XCD
-// when HG is a multiple of 8, and the query blocks reading that head's tiles share an L2.
-struct FlatBlock {
-    int qb, hg;
-};
-__device__ __forceinline__ FlatBlock flat_block() {
-    const int lin = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
-    return FlatBlock{lin / (int)gridDim.y, lin % (int)gridDim.y};
-}
 
 // QK: S^T[64 tok x 32 q] = K . Q^T + c0.  The two token blocks' accumulators are two
 // independent MFMA chains, started at c0 (minus the lane's running max, so the scores
@@ -188,17 +178,17 @@ __device__ __forceinline__ void pv_flat(const uint8_t* vt, int n, int hh, const 
 // The tile loop over tiles 0 .. T-1 (T a multiple of kFlatBufs).  The staging policy
 // `pol` provides
 //   kRing                      register slots of staged records in flight
-//   start(lds)                 loads and stages tiles 0 and 1, fills the slots
-//   stage(slot, buf, bias, x)  writes tile x from register slot `slot` into LDS and
-//                              refills the slot with tile x + kRing
+//   start(tm, lds)             loads and stages tiles 0 and 1, fills the slots
+//   stage(slot, buf, bias, x)  writes tile x from register slot `slot` into LDS
+//   refill(tm, slot, x)        loads tile x + kRing into the slot that tile x left
 //   tvalid(x)                  valid tokens of tile x (0 for an empty tile)
-//   mask(x, S)                 extra per-score masking of tile x (the causal chunk's
-//                              diagonal tile), a wave-uniform branch
+//   mask(x, S)                 extra per-score masking of tile x (chunk tiles that reach
+//                              past a query), a wave-uniform branch
 // and (m, l, acc) carry the online softmax of this wave's rows in and out.
 template <class Pol>
-__device__ __forceinline__ void flat_tiles(Pol& pol, const FlatWave& w, uint8_t* lds, const ph8 (&qf)[8],
+__device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const FlatWave& w, uint8_t* lds, const ph8 (&qf)[8],
                                            pf16v (&acc)[4], float& m, float& l, int T) {
-    pol.start(lds);
+    pol.start(tm, lds);
     flat_barrier();
     pf16v Sx[2][2];
     ph8 P[4];
@@ -266,27 +256,23 @@ __device__ __forceinline__ void flat_tiles(Pol& pol, const FlatWave& w, uint8_t*
                 __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            pol.refill(uu % Pol::kRing, t + 2);
+            pol.refill(tm, uu % Pol::kRing, t + 2);
             flat_barrier();
         }
     }
 }
 
-// Loads this wave's Q^T fragments (lane (query n, half hh), step s -> q[qrow][16s + 8hh
-// .. +8]) as fp16, each element times `mul` (1, or the fp16 factor folded into Q).
-__device__ __forceinline__ void flat_load_q(const PrefillParams& p, int b, int qh, bool ok, int qrow, int hh,
-                                            float mul, ph8 (&qf)[8]) {
-    const uint16_t* qp = p.q + (int64_t)b * p.q_sb + (int64_t)qh * p.q_sh + (int64_t)(ok ? qrow : 0) * p.q_st + 8 * hh;
+// Loads this wave's Q^T fragments (lane (query n, half hh), step s -> q[row][16s + 8hh
+// .. +8], `qp` the row) as fp16, each element times sm_scale x log2 e (one rounding).
+__device__ __forceinline__ void flat_load_q(const PrefillParams& p, const uint16_t* qp, bool ok, int hh, ph8 (&qf)[8]) {
     bool over = false;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-        pu4 w = ok ? *(const pu4*)(qp + 16 * s) : pu4{0u, 0u, 0u, 0u};
+        pu4 w = ok ? *(const pu4*)(qp + 8 * hh + 16 * s) : pu4{0u, 0u, 0u, 0u};
         if (p.q_bf16) w = bf16x8_to_f16(w, over);
         qf[s] = __builtin_bit_cast(ph8, w);
-        if (mul != 1.0f) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qf[s][e] = (_Float16)((float)qf[s][e] * mul);
-        }
+        for (int e = 0; e < 8; ++e) qf[s][e] = (_Float16)((float)qf[s][e] * p.scale_log2);
     }
     if (__ballot(over) && (threadIdx.x & 63) == 0 && p.err) atomicOr(p.err, HKV_ERR_BIT_RANGE);
 }

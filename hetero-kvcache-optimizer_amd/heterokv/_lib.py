@@ -154,6 +154,7 @@ SYMBOLS = [
     ("hkv_decode_attn", ctypes.c_int, [ctypes.POINTER(DecodeArgs), vp]),
     ("hkv_decode_attn_noalloc", ctypes.c_int, [ctypes.POINTER(DecodeArgs), vp]),
     ("hkv_prefill_workspace_bytes", ctypes.c_size_t, [i32, i32, i32]),
+    ("hkv_prefill_split_bytes", ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
     ("hkv_prefill_attn", ctypes.c_int, [ctypes.POINTER(PrefillArgs), vp]),
     ("hkv_pf_create", ctypes.c_int, [i32, ctypes.c_size_t, i32, ctypes.POINTER(vp)]),
     ("hkv_pf_destroy", ctypes.c_int, [vp]),

@@ -394,14 +394,19 @@ typedef struct HkvPrefillArgs {
     int32_t chunk_dtype;           /* F16 or BF16 */
     int32_t out_dtype;             /* F16 or BF16 */
     /* Needed with a causal chunk, or with INT4 tokens and zone tokens: the chunk's K/V
-     * are rewritten here in the zone layout, and the zone kernel leaves each query row's
-     * partial softmax state here for the INT4 kernel.  16-byte aligned,
-     * hkv_prefill_workspace_bytes() bytes; no zero fill needed.  NULL otherwise. */
+     * are rewritten here in the zone layout, and partial softmax states of the query rows
+     * are kept here.  16-byte aligned, hkv_prefill_workspace_bytes() bytes; no zero fill
+     * needed.  May be NULL otherwise.  With at least hkv_prefill_split_bytes() bytes, a
+     * call with too few query rows to fill the GPU also splits its keys over workgroups
+     * (any call; without the room it runs unsplit, with the same result up to rounding). */
     void* workspace;
     size_t workspace_bytes;
 } HkvPrefillArgs;
 
 size_t hkv_prefill_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t num_queries);
+/* Workspace bytes with which hkv_prefill_attn splits the keys of this call (its workspace
+ * fields are ignored); 0 if it would not split them. */
+size_t hkv_prefill_split_bytes(const HkvPrefillArgs* args);
 int hkv_prefill_attn(const HkvPrefillArgs* args, void* stream);
 
 /*

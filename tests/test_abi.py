@@ -277,3 +277,21 @@ def test_repack_and_zone_step_argument_errors(lib):
     z.tail_ring = 64
     z.hh_budget, z.hh_capacity = 32, 16             # heavy-hitter zone smaller than its budget
     _err(lib, lib.hkv_zone_step(ctypes.byref(z), None), -1, b"heavy-hitter")
+
+
+def test_prefill_split_rule(lib):
+    """Calls that fill the GPU, and short ones, are not split; a few queries over a long
+    history are, with the chunk's copy and a state row per piece row in the workspace."""
+    from heterokv import _lib
+
+    def split(hq, hkv, sq, int4, chunk=False):
+        a = _lib.PrefillArgs()
+        a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim, a.num_queries = 1, hq, hkv, 128, sq
+        a.int4_max_len = int4
+        a.chunk_k = a.chunk_v = 4096 if chunk else None
+        return lib.hkv_prefill_split_bytes(ctypes.byref(a))
+    assert split(32, 8, 2048, 131072) == 0 and split(32, 8, 64, 64) == 0
+    n = split(32, 8, 64, 32768, chunk=True)
+    chunk = 2 * 8 * 64 * 128 * 2
+    assert n > chunk and (n - chunk) % (8 * 256 * 132 * 4) == 0
+    assert lib.hkv_prefill_split_bytes(None) == 0

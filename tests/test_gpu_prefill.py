@@ -225,3 +225,64 @@ def test_random_geometries(seed):
     print("case: prefill seed %d B=%d %d/%d Sq=%d sink %d mids %s recents %s causal %s q_scale %g" % (
         seed, B, Hkv * nrep, Hkv, Sq, sink, mids, recents, causal, q_scale), flush=True)
     _case(2000 + seed, B, Hkv * nrep, Hkv, Sq, sink, mids, recents, causal=causal, q_scale=q_scale)
+
+
+# (B, Hq, Hkv, Sq, sink, mids, recents, causal): rows that end inside a unit of 256, units
+# that cross a group's heads, keys of one kind and of both, sequences without any key of a
+# kind, pieces of unequal length and a last one of a single token
+SPLIT_CASES = [
+    (1, 8, 2, 64, 16, [4000], [700], True),      # one whole unit per kv head, both kinds
+    (1, 8, 2, 65, 0, [4097], [0], False),        # INT4 only, one row past the unit, one token past a tile
+    (2, 14, 2, 37, 64, [3000, 0], [1500, 17], True),   # n_rep 7, a sequence without INT4 tokens
+    (2, 6, 2, 100, 0, [2500, 1], [0, 0], True),  # n_rep 3, a one-token INT4 zone
+    (1, 4, 4, 300, 64, [0], [4096], True),       # n_rep 1, fp16 keys only, two units
+    (1, 16, 1, 16, 0, [6000], [16], False),      # n_rep 16, exactly one unit
+]
+
+
+def _split_bytes(B, Hq, Hkv, Sq, sink, mid, recent, causal):
+    import ctypes
+    from heterokv import _lib
+    a = _lib.PrefillArgs()
+    a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim, a.num_queries = B, Hq, Hkv, 128, Sq
+    a.num_f16_zones = 2
+    a.f16[0] = _lib.F16Zone(k=None, v=None, capacity=sink + 16, max_len=sink, lens=None)
+    a.f16[1] = _lib.F16Zone(k=None, v=None, capacity=recent + 16, max_len=recent, lens=None)
+    a.int4_max_len = mid
+    a.chunk_k = a.chunk_v = 4096 if causal else None
+    return _lib.load().hkv_prefill_split_bytes(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES)
+def test_split_keys(case):
+    """Keys split over workgroups, against the float64 oracle; the size rule does split them."""
+    B, Hq, Hkv, Sq, sink, mids, recents, causal = case
+    assert _split_bytes(B, Hq, Hkv, Sq, sink, max(mids), max(recents), causal) > 0
+    print("case: prefill split %r" % (case,), flush=True)
+    _case(50 + SPLIT_CASES.index(case), B, Hq, Hkv, Sq, sink, mids, recents, causal=causal, poison=True)
+
+
+@pytest.mark.parametrize("hq,hkv,sq,io", [(32, 8, 203, torch.float16), (7, 1, 129, torch.bfloat16)])
+def test_split_matches_unsplit(hq, hkv, sq, io):
+    """The same call with a workspace of the documented size (no room to split) and with
+    its own: the same softmax over the same staged keys, so only the order of the float32
+    sums and the output's rounding differ (2 ulp of the output type at magnitude 1)."""
+    from heterokv import ops
+    from heterokv._lib import load
+    g = torch.Generator().manual_seed(77)
+    mid, rec = 9000, 1000
+    mk = lambda n: torch.randn((1, hkv, n, 128), generator=g).to(io).to(DEV)   # noqa: E731
+    pool = ops.Int4Pool((mid + 15) // 16, hkv, DEV)
+    bt = torch.arange((mid + 15) // 16, dtype=torch.int32, device=DEV)[None]
+    ops.pack_tokens(pool, mk(mid), mk(mid), 0, bt)
+    z = ops.F16Zone(1, hkv, rec, DEV)
+    z.write(mk(rec), mk(rec), 0)
+    q = torch.randn((1, hq, sq, 128), generator=g).to(io).to(DEV)
+    kw = dict(zones=[(z, None, rec)], pool=pool, block_table=bt, int4_max_len=mid, chunk_k=mk(sq), chunk_v=mk(sq))
+    ws = torch.empty(load().hkv_prefill_workspace_bytes(1, hq, sq), dtype=torch.uint8, device=DEV)
+    print("case: split vs unsplit", hq, hkv, sq, io, flush=True)
+    a = ops.prefill_attention(q, **kw).float()
+    b = ops.prefill_attention(q, workspace=ws, **kw).float()
+    torch.cuda.synchronize()
+    pool.check_errors()
+    assert (a - b).abs().max().item() <= 2 * (2.0 ** -10 if io == torch.float16 else 2.0 ** -7)
