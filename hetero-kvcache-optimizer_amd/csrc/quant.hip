@@ -426,6 +426,101 @@ __global__ __launch_bounds__(256) void dequantize_groups8_kernel(
     }
 }
 
+// Pool -> dequantized K and V of every token, [batch][H][T][128]: (code - zp) * scale in
+// float32, then the output dtype's rounding, as dequantize_groups does.  One wave per
+// (block, head) part of 2208 bytes; the whole op is one read of the records and one write
+// of the outputs, and the writes (79% of the bytes) bound it.  Lane i reads 4-byte code
+// words and writes 16-byte pieces that are consecutive over the lanes: K word i of a
+// 4-token group is token i / 16, dims 8 (i % 16) .. +7; for V, whose words hold four tokens
+// of one dim pair, lane (g, j) reads the eight words of its dims 8j .. 8j + 7 (each line is
+// read once into the L1) and keeps their four tokens' nibbles of its parity.
+// 28608 tokens x 8 heads, K and V (149 MB): 122 us as unpack + dequantize + stack per
+// tensor, 28.3 us here (5.3 TB/s, the rate of a large copy).
+struct DequantParams {
+    const uint8_t* pool;
+    int64_t pool_blocks;
+    const int32_t* bt;
+    int bt_stride, H, T, nblk;
+    void* k;
+    void* v;
+};
+
+// x s rounded to float32: the empty asm keeps the compiler from folding the product and the
+// fp16 conversion into one v_fma_mixlo_f16, which rounds once (and so differs from the
+// reference where the float32 product lies on an fp16 tie).
+__device__ __forceinline__ float mul_f32(float x, float s) {
+    float r = x * s;
+    asm("" : "+v"(r));
+    return r;
+}
+
+template <int kDtype>
+__device__ __forceinline__ void store8(void* out, int64_t i, const float (&x)[8]) {
+    if constexpr (kDtype == HKV_DTYPE_F32) {
+        float4* o = (float4*)((float*)out + i);
+        o[0] = make_float4(x[0], x[1], x[2], x[3]);
+        o[1] = make_float4(x[4], x[5], x[6], x[7]);
+    } else {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t a = kDtype == HKV_DTYPE_F16 ? f2h_rn(x[2 * e]) : f2bf_rn(x[2 * e]);
+            const uint32_t b = kDtype == HKV_DTYPE_F16 ? f2h_rn(x[2 * e + 1]) : f2bf_rn(x[2 * e + 1]);
+            w[e] = a | (b << 16);
+        }
+        *(uint4*)((uint16_t*)out + i) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+template <int kDtype>
+__global__ __launch_bounds__(256) void dequant_tokens_kernel(DequantParams p) {
+    touch_kernel_args(p);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int blk = (int)blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
+    if (blk >= p.nblk) return;
+    const int phys = load_uniform_i32(p.bt, (int64_t)b * p.bt_stride + blk);
+    if (phys < 0 || (int64_t)phys >= p.pool_blocks) return;
+    const uint8_t* part = p.pool + (int64_t)phys * RecordLayout(p.H).bytes + RecordLayout::part(h);
+    const int g = lane >> 4, j = lane & 15;
+    const uint32_t* kc = (const uint32_t*)(part + kPartKc);
+    const uint32_t* vc = (const uint32_t*)(part + kPartVc) + (g * 16 + 8 * (j & 1)) * 4 + (j >> 2);
+    const float* ks = (const float*)(part + kPartKs);
+    uint32_t kw[4], vw[8];
+    float ksc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {   // tokens 4i + g
+        kw[i] = kc[64 * i + lane];
+        ksc[i] = ks[4 * i + g];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) vw[e] = vc[4 * e];
+    const uint4 kz = *(const uint4*)(part + kPartKz);
+    const float4 vs4 = *(const float4*)(part + kPartVs + 16 * g);
+    const uint32_t vz = *(const uint32_t*)(part + kPartVz + 4 * g);
+    const float vs[4] = {vs4.x, vs4.y, vs4.z, vs4.w};
+    const uint32_t kzw[4] = {kz.x, kz.y, kz.z, kz.w};
+    const int64_t row0 = ((int64_t)b * p.H + h) * p.T + (int64_t)blk * kBlockTokens;
+    const int nv = min(kBlockTokens, p.T - blk * kBlockTokens);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float zp = (float)((kzw[i] >> (8 * g)) & 0xffu);
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = mul_f32((float)((kw[i] >> nib_shift(e)) & 0xFu) - zp, ksc[i]);
+        if (4 * i + g < nv) store8<kDtype>(p.k, (row0 + 4 * i + g) * kHeadDim + 8 * j, x);
+    }
+    const int par = 4 * ((j >> 1) & 1);   // dims 16 n + c, n = j / 2: the odd n are nibbles x4..x7
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float zp = (float)((vz >> (8 * t)) & 0xffu);
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = mul_f32((float)((vw[e] >> (nib_shift(t) + nib_shift(par))) & 0xFu) - zp, vs[t]);
+        if (4 * g + t < nv) store8<kDtype>(p.v, (row0 + 4 * g + t) * kHeadDim + 8 * j, x);
+    }
+}
+
 int grid_for(int64_t work, int per_block) {
     int64_t g = (work + per_block - 1) / per_block;
     if (g < 1) g = 1;
@@ -538,6 +633,35 @@ extern "C" int hkv_unpack_tokens(const uint8_t* pool, int64_t pool_blocks, const
                        (hipStream_t)stream, pool, pool_blocks, block_table, num_kv_heads, num_tokens,
                        which, codes, scales, zps);
     HKV_LAUNCH_CHECK("unpack_tokens_kernel");
+    return HKV_OK;
+}
+
+extern "C" int hkv_dequant_tokens(const uint8_t* pool, int64_t pool_blocks, const int32_t* block_table,
+                                  int32_t bt_stride, int32_t batch, int32_t num_kv_heads, int32_t head_dim,
+                                  int32_t num_tokens, void* out_k, void* out_v, int32_t out_dtype, void* stream) {
+    clear_error();
+    HKV_REQUIRE(head_dim == kHeadDim, HKV_ERR_UNSUPPORTED, "hkv_dequant_tokens: head_dim %d != 128", head_dim);
+    HKV_REQUIRE(out_dtype == HKV_DTYPE_F16 || out_dtype == HKV_DTYPE_BF16 || out_dtype == HKV_DTYPE_F32, HKV_ERR_ARG,
+                "hkv_dequant_tokens: unsupported dtype %d", out_dtype);
+    HKV_REQUIRE(batch >= 0 && num_kv_heads > 0 && num_tokens >= 0, HKV_ERR_ARG, "hkv_dequant_tokens: bad sizes");
+    if (batch == 0 || num_tokens == 0) return HKV_OK;
+    HKV_REQUIRE(pool && block_table && pool_blocks > 0 && out_k && out_v, HKV_ERR_ARG, "hkv_dequant_tokens: null pointer");
+    HKV_REQUIRE((((uintptr_t)pool | (uintptr_t)out_k | (uintptr_t)out_v) & 15) == 0, HKV_ERR_ARG,
+                "hkv_dequant_tokens: pool and outputs must be 16-byte aligned");
+    HKV_REQUIRE((int64_t)bt_stride * kBlockTokens >= num_tokens, HKV_ERR_CAPACITY,
+                "hkv_dequant_tokens: block table stride %d too small for %d tokens", bt_stride, num_tokens);
+    HKV_REQUIRE(batch <= 65535 && num_kv_heads <= 65535 && num_tokens <= (1 << 26), HKV_ERR_ARG,
+                "hkv_dequant_tokens: grid too large");
+    const int nblk = (int)(((int64_t)num_tokens + kBlockTokens - 1) / kBlockTokens);
+    const DequantParams p = {pool, pool_blocks, block_table, bt_stride, num_kv_heads, num_tokens, nblk, out_k, out_v};
+    const dim3 grid((unsigned)((nblk + 3) / 4), num_kv_heads, batch);
+    if (out_dtype == HKV_DTYPE_F16)
+        hipLaunchKernelGGL(dequant_tokens_kernel<HKV_DTYPE_F16>, grid, dim3(256), 0, (hipStream_t)stream, p);
+    else if (out_dtype == HKV_DTYPE_BF16)
+        hipLaunchKernelGGL(dequant_tokens_kernel<HKV_DTYPE_BF16>, grid, dim3(256), 0, (hipStream_t)stream, p);
+    else
+        hipLaunchKernelGGL(dequant_tokens_kernel<HKV_DTYPE_F32>, grid, dim3(256), 0, (hipStream_t)stream, p);
+    HKV_LAUNCH_CHECK("dequant_tokens_kernel");
     return HKV_OK;
 }
 

@@ -146,6 +146,7 @@ SYMBOLS = [
     ("hkv_pack_tokens", ctypes.c_int, [ctypes.POINTER(PackArgs), vp]),
     ("hkv_repack_codes", ctypes.c_int, [ctypes.POINTER(RepackArgs), vp]),
     ("hkv_unpack_tokens", ctypes.c_int, [vp, i64, vp, i32, i32, i32, i32, vp, vp, vp, vp]),
+    ("hkv_dequant_tokens", ctypes.c_int, [vp, i64, vp, i32, i32, i32, i32, i32, vp, vp, i32, vp]),
     ("hkv_zone_write", ctypes.c_int, [ctypes.POINTER(ZoneWriteArgs), vp]),
     ("hkv_zone_read", ctypes.c_int, [vp, vp, i32, i32, i32, i32, i32, vp, vp, vp]),
     ("hkv_zone_copy", ctypes.c_int, [vp, vp, i32, i32, vp, vp, i32, i32, i32, i32, i32, i32, vp]),

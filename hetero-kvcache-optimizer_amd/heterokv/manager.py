@@ -630,14 +630,8 @@ class HeteroKVManager:
         if st is None or st.int4_len == 0:
             return None, None, 0
         pool, bt = self._resident_view(st)
-        outs = []
-        for which in (0, 1):
-            per_b = []
-            for b in range(st.B):
-                c, s, z = ops.unpack_tokens(pool, bt[b], st.int4_len, which)
-                per_b.append(self._compressor.decompress(c, s, z, target_dtype=torch.float16))
-            outs.append(torch.stack(per_b))
-        return outs[0], outs[1], st.int4_len
+        k, v = ops.dequant_tokens(pool, bt[:st.B], st.int4_len)
+        return k, v, st.int4_len
 
     def _adaptive_selection(self, layer_idx: int, window_size: Optional[int]) -> List[str]:
         """The chunk keys manager.py:857-878 / :966-978 select: w = window_size, or the

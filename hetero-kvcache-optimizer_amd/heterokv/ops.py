@@ -281,6 +281,22 @@ def unpack_tokens(pool, block_table_row, num_tokens, which):
     return codes, scales, zps
 
 
+def dequant_tokens(pool, block_table, num_tokens, dtype=torch.float16):
+    """Pool -> dequantized (K, V) [B, H, T, 128] of the sequences of block_table [B, nblk]."""
+    dev = pool.device
+    if dtype not in _DTYPES:
+        raise HeteroKVError(-1, "dequant_tokens: unsupported dtype %s" % dtype)
+    bt = _i32(block_table, dev)
+    if bt.dim() == 1:
+        bt = bt.unsqueeze(0)
+    B, H = bt.shape[0], pool.num_kv_heads
+    k = torch.empty((B, H, num_tokens, HEAD_DIM), dtype=dtype, device=dev)
+    v = torch.empty_like(k)
+    check(load().hkv_dequant_tokens(_p(pool.data), pool.num_blocks, _p(bt), bt.shape[1], B, H, HEAD_DIM, num_tokens,
+                                    _p(k), _p(v), _DTYPES[dtype], stream_ptr(dev)), "hkv_dequant_tokens")
+    return k, v
+
+
 # ----------------------------------------------------------------------- fp16 zones
 class F16Zone:
     """fp16 zone storage: K [B, H, cap, 128] row-major, V in 16-token transposed tiles."""

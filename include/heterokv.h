@@ -199,6 +199,13 @@ int hkv_unpack_tokens(const uint8_t* pool, int64_t pool_blocks, const int32_t* b
                       int32_t num_kv_heads, int32_t head_dim, int32_t num_tokens,
                       int32_t which /* 0 = K, 1 = V */,
                       uint8_t* codes, float* scales, uint8_t* zps, void* stream);
+/* Pool -> dequantized tokens, as hkv_unpack_tokens + hkv_dequantize_groups give them
+ * ((code - zp) * scale in float32, rounded to out_dtype): tokens [0, num_tokens) of every
+ * sequence b (block table row b) to out_k / out_v [batch][num_kv_heads][num_tokens][128],
+ * 16-byte aligned, F16, BF16 or F32.  Tokens of a block with a bad id are not written. */
+int hkv_dequant_tokens(const uint8_t* pool, int64_t pool_blocks, const int32_t* block_table,
+                       int32_t bt_stride, int32_t batch, int32_t num_kv_heads, int32_t head_dim,
+                       int32_t num_tokens, void* out_k, void* out_v, int32_t out_dtype, void* stream);
 
 /*
  * Write `num_tokens` fp16 or bf16 tokens into an fp16 zone (sink / recent window /

@@ -266,3 +266,26 @@ def test_f16_zone_write_per_sequence_slots_and_uniform_base():
     assert torch.equal(z2.k, z3.k) and torch.equal(z2.v, z3.v)
     rk, _ = z2.read(16)
     assert torch.equal(rk[:, :, 11:16].cpu(), k)
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 65, 333])
+@pytest.mark.parametrize("H", [1, 3, 8])
+def test_dequant_tokens_is_unpack_plus_decompress(T, H):
+    """hkv_dequant_tokens against the unpack and dequantize kernels, bit for bit, with a NaN
+    row and every output dtype; the last block's tail and the tokens past T stay untouched."""
+    from heterokv import ops
+    print("case: dequant_tokens T=%d H=%d" % (T, H), flush=True)
+    nb = (T + 15) // 16
+    pool = ops.Int4Pool(2 * nb + 1, H, DEV)
+    bt = torch.randperm(2 * nb + 1, generator=torch.Generator().manual_seed(T))[:2 * nb].to(torch.int32).view(2, nb)
+    for b in range(2):
+        k, v = _rand_kv(100 * b + T, H, T)
+        k[0, 0, T // 2, 5] = float("nan")
+        ops.pack_tokens(pool, k.to(DEV), v.to(DEV), 0, bt[b:b + 1])
+    for dtype, bits in ((torch.float16, torch.int16), (torch.bfloat16, torch.int16), (torch.float32, torch.int32)):
+        got = ops.dequant_tokens(pool, bt, T, dtype)
+        for which in (0, 1):
+            for b in range(2):
+                exp = ops.dequantize_groups(*ops.unpack_tokens(pool, bt[b], T, which), dtype=dtype)
+                assert torch.equal(got[which][b].view(bits), exp.view(bits))
+    pool.check_errors()
