@@ -158,3 +158,22 @@ def test_cpu_tensor_is_rejected():
     from heterokv import HeteroKVError, KVCompressor
     with pytest.raises(HeteroKVError):
         KVCompressor().compress(torch.zeros(128, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("G", [8, 16, 64, 128, 256, 512, 96, 1024])
+@pytest.mark.parametrize("n", [8, 120, 128 * 37, 128 * 37 + 8, 4099])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_group_lanes_match_oracle(G, n, dtype):
+    """Groups of 8 << k values (several lanes per group, short last groups), beside sizes the
+    one-wave-per-group kernel takes (96, 1024, n not a multiple of 8, an unaligned view)."""
+    from heterokv import KVCompressor
+    g = torch.Generator().manual_seed(G * 7 + n)
+    x = (torch.randn(n + 1, generator=g) * 3).to(dtype)
+    x[n // 2] = 60.0
+    for off in (0, 1):
+        xd = x.to(DEV)[off:off + n]
+        codes, scales, zps = KVCompressor(group_size=G).compress(xd)
+        rc, rs, rz = oc.compress(x[off:off + n].float().numpy(), G)
+        assert np.array_equal(codes.cpu().numpy(), rc)
+        assert np.array_equal(scales.cpu().numpy().view(np.uint32), rs.view(np.uint32))
+        assert np.array_equal(zps.cpu().numpy(), rz)
