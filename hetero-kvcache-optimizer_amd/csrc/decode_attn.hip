@@ -18,8 +18,9 @@
 // pair (1024 + zp) leaves the exact integer code - zp.  The K scale multiplies
 // the score, the V scale multiplies the probability, both in fp32.
 //
-// Work split.  Every (sequence, kv head) pair is cut into S byte-balanced
-// ranges (S chosen so that S x pairs is about one workgroup per CU); a range is
+// Work split.  Every (sequence, kv head) pair is cut into S cost-balanced
+// ranges (S such that the grid fits the CUs once, choose_ranges; in a ragged batch
+// by the sequences' lengths, share_ranges); a range is
 // a run of items in the order [INT4 blocks | fp16 zone tiles], and each of the
 // 8 waves of the workgroup takes a contiguous piece of it.  Waves merge through
 // LDS, workgroups through a workspace: the last workgroup of a pair to finish
@@ -73,7 +74,7 @@ constexpr int kPrefetch = HKV_DECODE_PREFETCH;  // INT4 block pairs in flight pe
 #define HKV_DECODE_F16_DEPTH 1
 #endif
 constexpr int kF16Depth = HKV_DECODE_F16_DEPTH;
-constexpr int kMaxSplits = 64;
+constexpr int kMaxSplits = 64;           // the slice merge takes 16 x 4 states
 constexpr int kLineWords = 64;           // ints per 256-byte hand-off line
 // Slice merge: the pair's arrival word holds the arrivals of the current launch in bits
 // 0-15, a generation in bits 16-29 that the last arrival advances (clearing the count),
@@ -134,6 +135,7 @@ constexpr int64_t kF16ItemBytes = kBlockTokens * kHeadDim * 2 * 2;           // 
 #define HKV_INT4_COST 3300
 #endif
 constexpr int64_t kInt4Cost = HKV_INT4_COST;
+constexpr float kStartCost = 16384.0f;
 
 struct ZoneP {
     const uint16_t* k;
@@ -169,12 +171,14 @@ struct DecodeParams {
     unsigned* owners;         // agent-scope XCD mask (placement check): word 1 of the same line
     int* counters_l2;         // XCD-local line: [0] slice-merge arrivals, [1] ticket
     float* partials;
-    int max_splits;
+    int max_splits;            // ranges per pair (p.lin_ranges == 0)
+    int lin_ranges;            // > 0: ranges per kv head over all sequences, shared out by their lengths
+    int split_stride;          // floats between the partial states of consecutive shared-out ranges
+    int slice_outputs;         // slice merge: outputs per slice, ceil(n_rep * 128 / max_splits)
     int64_t part_pair_stride;  // floats between the partial blocks of consecutive pairs (256-byte multiple)
     int xcc_local;             // 1: all ranges of a pair run on one XCD (see above)
     int nxcc;                  // XCDs the dispatcher round-robins over
     int coop;                  // 1: slice merge by every range of a pair (see the kernel's tail)
-    int slice_outputs;         // slice merge: outputs per slice, ceil(n_rep * 128 / ranges)
     unsigned long long merge_wait;   // slice merge: constant-clock ticks a range waits for the others
     // optional score output (kScores): row (b, q head) holds the log2-domain score of
     // every item [INT4 tokens | zone 0 | zone 1 | zone 2]; zone z starts at sc_zone[z]
@@ -216,19 +220,54 @@ __device__ __forceinline__ f2 ld_l2_f2(__amdgpu_buffer_rsrc_t r, int byte_off) {
 // The same loads at device scope (sc1: coherent with other XCDs' device-scope stores).
 constexpr int kAuxL2 = 1, kAuxDevice = 16;
 
-// Slice merge: the (m, l) pair and output d of eight partial states (splits q + base,
-// q + base + 4, ...), with loads of cache policy kAux.
-template <int kAux>
-__device__ __forceinline__ void load_slice8(__amdgpu_buffer_rsrc_t prs, int q, int base, int nsplit, int nrep, int hd,
-                                            int d, float (&ms)[8], float (&ls)[8], float (&os)[8]) {
+// The value of a lane exchanged within its 16-lane row, x = 1, 2 (the lane ^ x of the
+// quad), 4 (the mirrored lane of the half row: the other quad) or 8 (of the row: the other
+// half); every lane of the row must be active.
+__device__ __forceinline__ float row_xchg(float v, int x) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, x == 1   ? __builtin_amdgcn_mov_dpp(i, 0xB1, 0xF, 0xF, false)
+                                     : x == 2 ? __builtin_amdgcn_mov_dpp(i, 0x4E, 0xF, 0xF, false)
+                                     : x == 4 ? __builtin_amdgcn_mov_dpp(i, 0x141, 0xF, 0xF, false)
+                                              : __builtin_amdgcn_mov_dpp(i, 0x140, 0xF, 0xF, false));
+}
+
+// Slice merge: the softmax state (M, L, O) of output d of head hd from all nsplit <= kLanes
+// kPer partial states, kLanes consecutive lanes per output, lane q taking states q, q +
+// kLanes, ... (all their loads in flight together, of cache policy kAux), then the lanes
+// merging in a fixed order.
+template <int kAux, int kLanes, int kPer>
+__device__ __forceinline__ void merge_states(__amdgpu_buffer_rsrc_t prs, int q, int nsplit, int sstride, int hd, int d,
+                                             float& M, float& L, float& O) {
+    float ms[kPer], ls[kPer], os[kPer];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int sj = q + base + 4 * j;
-        const int off = min(sj, nsplit - 1) * (nrep * kPartStride) + hd * kPartStride;
+    for (int j = 0; j < kPer; ++j) {
+        const int sj = q + kLanes * j;
+        const int off = min(sj, nsplit - 1) * sstride + hd * kPartStride;
         const f2 ml = __builtin_bit_cast(f2, __builtin_amdgcn_raw_buffer_load_b64(prs, (off + kHeadDim) * 4, 0, kAux));
         ms[j] = sj < nsplit ? ml.x : -INFINITY;
         ls[j] = ml.y;
         os[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(prs, (off + d) * 4, 0, kAux));
+    }
+    M = ms[0];
+#pragma unroll
+    for (int j = 1; j < kPer; ++j) M = fmaxf(M, ms[j]);
+    L = 0.f;
+    O = 0.f;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const float e = (ms[j] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ms[j] - M);
+        O += os[j] * e;
+        L += ls[j] * e;
+    }
+#pragma unroll
+    for (int x = 1; x < kLanes; x <<= 1) {
+        const float M2 = row_xchg(M, x), L2 = row_xchg(L, x), O2 = row_xchg(O, x);
+        const float Mn = fmaxf(M, M2);
+        const float a = (M == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
+        const float c = (M2 == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M2 - Mn);
+        O = O * a + O2 * c;
+        L = L * a + L2 * c;
+        M = Mn;
     }
 }
 
@@ -275,14 +314,6 @@ __device__ __forceinline__ int slice_arrival(int* arrived, int nsplit, unsigned 
 }
 
 __device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
-
-// The value of lane (lane ^ x) of the same quad, x = 1 or 2 (DPP quad_perm [1,0,3,2] or
-// [2,3,0,1]); every lane of the quad must be active.
-__device__ __forceinline__ float quad_xor(float v, int x) {
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, x == 1 ? __builtin_amdgcn_mov_dpp(i, 0xB1, 0xF, 0xF, false)
-                                            : __builtin_amdgcn_mov_dpp(i, 0x4E, 0xF, 0xF, false));
-}
 
 struct Int4Blk {
     u4 k;         // K codes of token (lane%16), dims 32g..32g+31
@@ -602,8 +633,9 @@ __device__ __forceinline__ int next_unit(int* ctr, int& seq) {
 
 // Splits that stream only INT4 blocks when a pair's ranges are made of one kind
 // each, or 0 when every range takes the same share of both kinds.  Ranges of one
-// kind avoid a second pipeline start inside a range; they are used when the
-// rounding of nsplit into two groups costs at most ~6% over an even share.  Costs:
+// kind avoid a second pipeline start inside a range, ~1 us; they are used when the
+// rounding of nsplit into two groups costs at most ~6%, or kStartCost (about what a
+// range streams in that time), over an even share.  Costs:
 // an INT4 block counts kInt4Cost bytes (its 2208 bytes, plus the block-id
 // indirection and the nibble decode), an fp16 tile its 8192 bytes.
 //
@@ -615,7 +647,70 @@ __device__ __forceinline__ int int4_splits(int nb4, int ntf, int nsplit) {
     int s4 = (int)(c4 * (float)nsplit / ct + 0.5f);
     s4 = min(max(s4, 1), nsplit - 1);
     const float worst = fmaxf(c4 / (float)s4, cf / (float)(nsplit - s4));
-    return worst * 16.0f <= ct / (float)nsplit * 17.0f ? s4 : 0;
+    const float share = ct / (float)nsplit;
+    return worst <= fmaxf(share * (17.0f / 16.0f), share + kStartCost) ? s4 : 0;
+}
+
+// The range of one kv head's run of p.lin_ranges ranges, shared out over the sequences by
+// their lengths: sequence b gets ceil(cost_b / t) ranges, for the smallest t (by bisection)
+// with which all fit, so no range is longer than t.  With the same number of ranges for
+// every sequence, the longest one's set the time of a ragged batch.  Lane b works on
+// sequence b (B <= 64, checked on the host); every wave finds the same plan.
+struct RangePlan {
+    int b, split, nsplit, first;   // sequence, range within it, its ranges (0: none), the first one's index
+};
+__device__ __forceinline__ RangePlan share_ranges(const DecodeParams& p, int lin) {
+    const int lane = threadIdx.x & 63, n = p.lin_ranges;
+    float cost = 0.f;
+    if (lane < p.B) {
+        const int len4 = p.int4_lens ? min(max(p.int4_lens[lane], 0), p.int4_max_len) : p.int4_max_len;
+        int tiles = 0;
+#pragma unroll
+        for (int zi = 0; zi < HKV_MAX_F16_ZONES; ++zi)
+            if (zi < p.nz) {
+                const int l = p.z[zi].lens ? min(max(p.z[zi].lens[lane], 0), p.z[zi].max_len) : p.z[zi].max_len;
+                tiles += (l + kBlockTokens - 1) / kBlockTokens;
+            }
+        cost = (float)((len4 + kBlockTokens - 1) / kBlockTokens) * (float)kInt4Cost + (float)tiles * (float)kF16ItemBytes;
+    }
+    // lane moves only, no LDS permutes (which made this plan 2.5 us long); every lane adds the
+    // same pairs, so all get the same bits
+    const auto wave_sum = [](float v) {
+#pragma unroll
+        for (int x = 1; x < 16; x <<= 1) v += row_xchg(v, x);
+        const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+        const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
+    };
+    const float total = wave_sum(cost);
+    // sum of ceil(cost / t) <= total / t + B: t = total / (n - B) fits
+    float lo = total / (float)n, hi = total / (float)(n > p.B ? n - p.B : 1);
+    const auto ranges = [&](float t) {
+        const float r = ceilf(cost / t);   // 0 / 0 (no key at all) counts as one range
+        return lane < p.B ? (r > 1.f ? (r < (float)kMaxSplits ? r : (float)kMaxSplits) : 1.f) : 0.f;
+    };
+    if (n <= p.B) hi = INFINITY;           // one range each
+    else
+#pragma unroll 1
+        for (int i = 0; i < 5; ++i) {
+            const float mid = 0.5f * (lo + hi);
+            if (wave_sum(ranges(mid)) <= (float)n) hi = mid;
+            else lo = mid;
+        }
+    const int mine = (int)ranges(hi);
+    int end = mine;                        // inclusive scan over the lanes
+    end += __builtin_amdgcn_update_dpp(0, end, 0x111, 0xF, 0xF, false);   // row_shr 1, 2, 4, 8: within rows of 16
+    end += __builtin_amdgcn_update_dpp(0, end, 0x112, 0xF, 0xF, false);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x114, 0xF, 0xF, false);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x118, 0xF, 0xF, false);
+    const int r0 = __builtin_amdgcn_readlane(end, 15), r1 = __builtin_amdgcn_readlane(end, 31),
+              r2 = __builtin_amdgcn_readlane(end, 47);
+    end += lane < 16 ? 0 : lane < 32 ? r0 : lane < 48 ? r0 + r1 : r0 + r1 + r2;
+    const int b = __builtin_popcountll(__ballot(lane < p.B && end <= lin));   // sequences that end at or before lin
+    if (b >= p.B) return RangePlan{0, 0, 0, 0};
+    const int last = __builtin_amdgcn_readlane(end, b), cnt = __builtin_amdgcn_readlane(mine, b);
+    return RangePlan{b, lin - (last - cnt), cnt, last - cnt};
 }
 
 // floor(n i / d) for the range bounds: n < 2^22 items (host-checked), i <= d <= 64,
@@ -630,11 +725,11 @@ __device__ __forceinline__ int part_point(int n, int i, int d) {
 // hand-off (group-scope buffer loads), else agent-scope loads.
 template <bool kL2>
 __device__ __forceinline__ void load_partials(__amdgpu_buffer_rsrc_t prs, const float* parts, int s0, int K,
-                                              int nsplit, int nrep, int hd, int d4, float* ms, float* ls, f4* os) {
+                                              int nsplit, int sstride, int hd, int d4, float* ms, float* ls, f4* os) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int sj = s0 + j * K;
-        const int off = min(sj, nsplit - 1) * (nrep * kPartStride) + hd * kPartStride;
+        const int off = min(sj, nsplit - 1) * sstride + hd * kPartStride;
         if constexpr (kL2) {
             const f2 ml = ld_l2_f2(prs, (off + kHeadDim) * 4);   // m, l side by side (8-byte aligned)
             ms[j] = sj < nsplit ? ml.x : -INFINITY;
@@ -650,15 +745,28 @@ __device__ __forceinline__ void load_partials(__amdgpu_buffer_rsrc_t prs, const 
 }
 
 // kL2: the XCD-local hand-off (p.xcc_local), a template parameter so that each hand-off's
-// kernel carries only its own tail code.
-template <bool kDynamic, bool kScores, bool kL2>
+// kernel carries only its own tail code.  kShared: p.lin_ranges > 0, for the same reason
+// (in one kernel with it, the 32K decode's launch was 0.25 us longer).
+template <bool kDynamic, bool kScores, bool kL2, bool kShared>
 __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     touch_kernel_args(p);   // the range plan below reads the arguments in a dependent chain
-    const int BH = p.B * p.Hkv;
-    const int bh = blockIdx.x % BH;
-    const int split = blockIdx.x / BH;
-    const int nsplit = p.max_splits;
-    const int b = bh / p.Hkv, h = bh % p.Hkv;
+    int b, h, split, nsplit, first = 0;
+    if constexpr (kShared) {
+        const RangePlan r = share_ranges(p, (int)blockIdx.x / p.Hkv);
+        if (r.nsplit == 0) return;   // a range left over
+        b = r.b;
+        h = (int)blockIdx.x % p.Hkv;
+        split = r.split;
+        nsplit = r.nsplit;
+        first = r.first;
+    } else {
+        const int BH = p.B * p.Hkv, pair = blockIdx.x % BH;
+        b = pair / p.Hkv;
+        h = pair % p.Hkv;
+        split = blockIdx.x / BH;
+        nsplit = p.max_splits;
+    }
+    const int bh = b * p.Hkv + h;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: buffer resources stay scalar
     const int c = lane & 15, g = lane >> 4;
@@ -900,7 +1008,7 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     // the path that skips the OR, the compiler waited for all loads, the OR included,
     // before the first shuffle of the merge.
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    if (kL2 && threadIdx.x == 0) {
+    if (kL2 && nsplit > 1 && threadIdx.x == 0) {   // one range hands nothing off: no bit left behind
         owner_bit = 1u << (__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15);
         owner_old = __hip_atomic_fetch_or(&p.owners[bh * kLineWords], owner_bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -935,12 +1043,16 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     const int nout = nrep * kHeadDim;
     // the pair's partial states, computed once and held in registers (opaque to the
     // compiler, which would otherwise read the arguments again after the arrival wait)
-    float* parts = p.partials + (int64_t)bh * p.part_pair_stride;
+    // (shared-out ranges: numbered per kv head, over all sequences)
+    float* parts = p.partials + (kShared ? (int64_t)(h * p.lin_ranges + first) * p.split_stride
+                                                  : (int64_t)bh * p.part_pair_stride);
     uint16_t* obase = p.out + (int64_t)b * p.o_sb + (int64_t)(h * nrep) * p.o_sh;   // this kv head's outputs
     int64_t osh = p.o_sh;
-    int obf16 = p.out_bf16, slice_outputs = p.slice_outputs;
-    asm volatile("" : "+s"(parts), "+s"(obase), "+s"(osh), "+s"(obf16), "+s"(slice_outputs));
-    float* part = parts + (int64_t)split * (nrep * kPartStride);
+    // slice merge: outputs per slice
+    int obf16 = p.out_bf16, slice_outputs = kShared ? (nout + nsplit - 1) / nsplit : p.slice_outputs;
+    int sstride = kShared ? p.split_stride : nrep * kPartStride;
+    asm volatile("" : "+s"(parts), "+s"(obase), "+s"(osh), "+s"(obf16), "+s"(slice_outputs), "+s"(sstride));
+    float* part = parts + (int64_t)split * sstride;
     for (int idx = threadIdx.x; idx < nout; idx += kThreads) {
         const int hd = idx >> 7, d = idx & (kHeadDim - 1);
         float M = -INFINITY;
@@ -988,7 +1100,9 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
-    if (p.coop) {
+    // (shared-out ranges: all resident; XCD-local ones of fewer than n_rep ranges, with more
+    // than 128 outputs per slice, are quicker through the last arrival)
+    if (kShared ? !kL2 || nsplit >= nrep : p.coop != 0) {
         // ---- slice merge (every range of the pair resident; atomics and loads in the
         // XCD's L2 with the XCD-local hand-off, at device scope otherwise).  Each
         // range adds itself to the pair's arrival count, waits until the count is complete
@@ -1022,55 +1136,26 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
             TL_FLUSH(tl_info);
             return;
         }
-        // slice sl = outputs [sl S, sl S + S) of the pair's nout (head-major: head, dim);
-        // 4 threads per output, thread q of an output taking splits q, q + 4, ...
+        // slice sl = outputs [sl S, sl S + S) of the pair's nout (head-major: head, dim).  Up
+        // to 32 states, 4 lanes per output load 8 each; beyond, 16 lanes load 4 each, where 4
+        // lanes took a second load round trip (64 device-scope states, one sequence of 28/4
+        // heads at 32K: 14.1 -> 13.4 us; 16 lanes for 32 XCD-local states cost 0.15 us)
         const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)parts, 0, (int)(nsplit * nrep * kPartStride * sizeof(float)), 0x00020000);
+            (void*)parts, 0, (int)(nsplit * sstride * sizeof(float)), 0x00020000);
         const int S = slice_outputs;
         const int sl0 = slices == 2 ? 0 : split, sl1 = slices == 2 ? nsplit : split + 1;
+        const int lsh = nsplit > 32 ? 4 : 2;
         for (int sl = sl0; sl < sl1; ++sl) {
-            for (int t = threadIdx.x; t < 4 * S; t += kThreads) {
-                const int o = sl * S + (t >> 2), q = t & 3;
-                const bool live = o < nout;
+            for (int t = threadIdx.x; t < S << lsh; t += kThreads) {
+                const int o = sl * S + (t >> lsh), q = t & ((1 << lsh) - 1);
                 const int hd = min(o, nout - 1) >> 7, d = min(o, nout - 1) & (kHeadDim - 1);
-                float M = -INFINITY, L = 0.f, O = 0.f;
-                for (int base = 0; q + base < nsplit; base += 32) {
-                    float ms[8], ls[8], os[8];
-                    if (kL2)
-                        load_slice8<kAuxL2>(prs, q, base, nsplit, nrep, hd, d, ms, ls, os);
-                    else
-                        load_slice8<kAuxDevice>(prs, q, base, nsplit, nrep, hd, d, ms, ls, os);
-                    float Mc = ms[0];
-#pragma unroll
-                    for (int j = 1; j < 8; ++j) Mc = fmaxf(Mc, ms[j]);
-                    if (Mc > -INFINITY) {
-                        const float Mn = fmaxf(M, Mc);
-                        const float a = (M == -INFINITY) ? 0.f : fast_exp2(M - Mn);
-                        float Oc = 0.f, Lc = 0.f;
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            const float e = (ms[j] == -INFINITY) ? 0.f : fast_exp2(ms[j] - Mn);
-                            Oc += os[j] * e;
-                            Lc += ls[j] * e;
-                        }
-                        O = O * a + Oc;
-                        L = L * a + Lc;
-                        M = Mn;
-                    }
-                }
-                // the output's four threads are one quad of lanes: exchanged with DPP quad
-                // permutes (lane ^ 1, then lane ^ 2), no LDS round trip
-#pragma unroll
-                for (int x = 1; x < 4; x <<= 1) {
-                    const float M2 = quad_xor(M, x), L2 = quad_xor(L, x), O2 = quad_xor(O, x);
-                    const float Mn = fmaxf(M, M2);
-                    const float a = (M == -INFINITY) ? 0.f : fast_exp2(M - Mn);
-                    const float c = (M2 == -INFINITY) ? 0.f : fast_exp2(M2 - Mn);
-                    O = O * a + O2 * c;
-                    L = L * a + L2 * c;
-                    M = Mn;
-                }
-                if (live && q == 0) {
+                constexpr int kAux = kL2 ? kAuxL2 : kAuxDevice;
+                float M, L, O;
+                if (lsh == 4)
+                    merge_states<kAux, 16, 4>(prs, q, nsplit, sstride, hd, d, M, L, O);
+                else
+                    merge_states<kAux, 4, 8>(prs, q, nsplit, sstride, hd, d, M, L, O);
+                if (o < nout && q == 0) {
                     const float r = L > 0.f ? O / L : 0.f;
                     obase[(int64_t)hd * osh + d] = obf16 ? f2bf_rn(r) : f2h_rn(r);
                     if (kScores && d == 0) {
@@ -1120,7 +1205,7 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     // s = k, k + K, k + 2K, ... (K = threads per unit); all its loads are
     // independent.  The K per-thread states then merge through LDS.
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)parts, 0, (int)(nsplit * nrep * kPartStride * sizeof(float)), 0x00020000);
+        (void*)parts, 0, (int)(nsplit * sstride * sizeof(float)), 0x00020000);
     const int units = nrep * (kHeadDim / 4);
     const int K = kThreads / units;                  // >= 1 because nrep <= 16
     float* sm = smem;                                // [K][units][6] = (M, L, O[4])
@@ -1133,9 +1218,9 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
             float ms[8], ls[8];
             f4 os[8];
             if (kL2)
-                load_partials<true>(prs, parts, s0, K, nsplit, nrep, hd, d4, ms, ls, os);
+                load_partials<true>(prs, parts, s0, K, nsplit, sstride, hd, d4, ms, ls, os);
             else
-                load_partials<false>(prs, parts, s0, K, nsplit, nrep, hd, d4, ms, ls, os);
+                load_partials<false>(prs, parts, s0, K, nsplit, sstride, hd, d4, ms, ls, os);
             // the eight states merge with independent terms against their common max
             float Mc = ms[0];
 #pragma unroll
@@ -1225,19 +1310,66 @@ int num_cus() {
     return n;
 }
 
-// Ranges per (sequence, kv head): about one 8-wave workgroup per CU for the
-// whole launch, each reading at least ~96 KB, at most kMaxSplits.
-int choose_splits(int BH, int int4_max_len, const int32_t* f16_max_lens, int nz, int hint) {
-    if (hint > 0) return hint < kMaxSplits ? hint : kMaxSplits;
+// Ranges.  A workgroup of 8 waves fills a CU (208 VGPRs), so the grid takes at most one
+// workgroup per CU when the pairs leave room for that: one workgroup more runs as a second
+// round (3 sequences of 32/8 heads at 32K: 11 ranges per pair, 264 workgroups, 44.7 us; 10
+// ranges 28.8 us).  Within that, a range holds at least two units (an fp16 tile or a pair of
+// INT4 blocks), since a short range costs little and the slice merge needs at least n_rep
+// ranges (507 tokens of 32/8 heads: 3 ranges of ~96 KB 8.8 us, 16 ranges 6.9 us, 32 ranges
+// 7.1 us; 28/4 heads 12.4, 8.4 and 8.4 us).  Few units stay in one range, without a
+// hand-off: up to kOneRange, two per wave (164 tokens: 5.9 us against 6.8 us), and with the
+// dearer last-arrival merge of fewer than n_rep ranges while s ranges take no more than
+// kOneRangeWide units off one (units (s - 1) / s; pairs for two ranges each, n_rep 4 to 8: 36
+// units 9.9 - 10.9 us in one, 10.5 - 11.2 in two; 49 units 14.4 - 15.1 and 13.4 - 13.9).
+// Where one round leaves CUs idle that two rounds would use, ranges still long in two (kLongRange bytes) take two (3 sequences of
+// 32/32 heads of 14K to 33K tokens: 2 ranges, 192 workgroups, 106 us; 5 ranges 96 us).
+// Sequences with lengths of their own share the ranges out by length (share_ranges) where an
+// even share is long: the plan costs a range ~1 us, and with kv heads that are no multiple
+// of the XCDs the XCD-local hand-off too.  8 sequences of 32/8 heads of 7K to 33K tokens
+// 60.6 -> 51.2 us, 5 of them 42.1 -> 36.1, 3 of 32/32 heads 102 -> 84; of 2K to 9K tokens
+// (even shares of 410 KB) 8 of 32/8 heads 23.2 -> 23.0 and 16 of 28/4 heads 24.6 -> 27.0.
+constexpr int kOneRange = 16, kOneRangeWide = 22;
+constexpr int64_t kLongRange = 512 * 1024;
+
+struct Ranges {
+    int per_pair;   // ranges per (sequence, kv head) pair, or
+    int lin;        // > 0: ranges per kv head, shared out over the sequences
+};
+
+Ranges choose_ranges(int B, int Hkv, int nrep, int int4_max_len, int64_t int4_item_bytes, const int32_t* f16_max_lens, int nz,
+                     bool own_lens, int hint) {
+    if (hint > 0) return Ranges{hint < kMaxSplits ? hint : kMaxSplits, 0};
+    const int64_t BH = (int64_t)B * Hkv, cus = num_cus();
+    int64_t units = ((int64_t)int4_max_len + 2 * kBlockTokens - 1) / (2 * kBlockTokens);
+    int64_t bytes = ((int64_t)int4_max_len + kBlockTokens - 1) / kBlockTokens * int4_item_bytes;
+    for (int i = 0; i < nz; ++i) {
+        const int64_t t = ((int64_t)f16_max_lens[i] + kBlockTokens - 1) / kBlockTokens;
+        units += t;
+        bytes += t * kF16ItemBytes;
+    }
+    const int64_t by_units = (units + 1) / 2 > nrep ? (units + 1) / 2 : nrep;
+    const int64_t one = cus / BH, two = 2 * cus / BH;
+    if (units <= kOneRange || (one < nrep && units * (one - 1) <= kOneRangeWide * one)) return Ranges{1, 0};
+    if (own_lens && B > 1 && B <= 64 && cus / Hkv >= B && bytes >= (one > 0 ? one : 1) * kLongRange) {
+        const int64_t lin = cus / Hkv < B * by_units ? cus / Hkv : B * by_units;
+        if (lin > B) return Ranges{1, (int)lin};
+    }
+    int64_t s = one;
+    if (two * 100 > 115 * 2 * one && bytes >= two * kLongRange) s = two;
+    if (s > kMaxSplits) s = kMaxSplits;
+    if (s > by_units) s = by_units;
+    return Ranges{(int)(s < 1 ? 1 : s), 0};
+}
+
+// The fewest ranges a call without a hint may be cut to when its workspace is smaller than
+// the documented size: about one workgroup per CU, each reading at least ~96 KB.
+int least_splits(int BH, int int4_max_len, const int32_t* f16_max_lens, int nz) {
     int64_t bytes = (int64_t)((int4_max_len + kBlockTokens - 1) / kBlockTokens) * kInt4ItemBytes;
     for (int i = 0; i < nz; ++i) bytes += (int64_t)((f16_max_lens[i] + kBlockTokens - 1) / kBlockTokens) * kF16ItemBytes;
-    const int cus = num_cus();
-    int64_t s = (cus + BH - 1) / BH;                       // fill the chip once
+    int64_t s = (num_cus() + BH - 1) / BH;
     const int64_t by_size = (bytes + 96 * 1024 - 1) / (96 * 1024);
-    if (s > by_size) s = by_size;                           // small problems: fewer, fuller ranges
-    if (s < 1) s = 1;
-    if (s > kMaxSplits) s = kMaxSplits;
-    return (int)s;
+    if (s > by_size) s = by_size;
+    return (int)(s < 1 ? 1 : s > kMaxSplits ? kMaxSplits : s);
 }
 
 // Workspace: [header (error word) | agent lines (ticket, XCD mask) | XCD-local lines
@@ -1261,6 +1393,12 @@ size_t workspace_bytes(int B, int Hq, int Hkv, int nsplit) {
     const size_t BH = (size_t)B * Hkv;
     const int nrep = Hq / Hkv;
     return kTicketAreaEnd + BH * pair_part_bytes(nrep, nsplit);
+}
+
+// With shared-out ranges: one partial state per range, each on lines of its own.
+int split_stride_floats(int nrep) { return (int)(align256((size_t)nrep * kPartStride * sizeof(float)) / sizeof(float)); }
+size_t shared_workspace_bytes(int Hkv, int nrep, int lin) {
+    return kTicketAreaEnd + (size_t)Hkv * lin * split_stride_floats(nrep) * sizeof(float);
 }
 
 // XCDs that workgroups are dispatched over round-robin: gfx950 has 32 CUs per
@@ -1380,11 +1518,24 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
                 "hkv_decode_attn: fp16 zones hold more than %d tokens", kMaxZoneTokens);
     const int64_t BH = (int64_t)a->batch * a->num_kv_heads;
     HKV_REQUIRE(BH < 65536, HKV_ERR_ARG, "hkv_decode_attn: batch x kv heads too large");
-    const int ms = choose_splits((int)BH, a->int4_max_len, zl, a->num_f16_zones, a->splits_hint);
+    bool own_lens = a->int4_lens != nullptr;
+    for (int i = 0; i < a->num_f16_zones; ++i) own_lens = own_lens || a->f16[i].lens != nullptr;
+    const Ranges rg = choose_ranges(a->batch, a->num_kv_heads, nrep, a->int4_max_len, kInt4ItemBytes, zl,
+                                    a->num_f16_zones, own_lens, a->splits_hint);
+    int ms = rg.per_pair, lin = rg.lin;
+    if (a->splits_hint <= 0) {
+        const int least = least_splits((int)BH, a->int4_max_len, zl, a->num_f16_zones);
+        if (lin > 0 && shared_workspace_bytes(a->num_kv_heads, nrep, lin) > ws_bytes) {
+            lin = 0;
+            ms = least;
+        }
+        while (ms > least && workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, ms) > ws_bytes) --ms;
+    }
     HKV_REQUIRE(ms == 1 || BH <= kHandoffPairs, HKV_ERR_CAPACITY,
                 "hkv_decode_attn: %d ranges per pair for %lld (sequence, kv head) pairs; a split launch hands off "
                 "at most %lld pairs", ms, (long long)BH, (long long)kHandoffPairs);
-    const size_t need = workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, ms);
+    const size_t need = lin > 0 ? shared_workspace_bytes(a->num_kv_heads, nrep, lin)
+                                : workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, ms);
     HKV_REQUIRE(ws_bytes >= need, HKV_ERR_CAPACITY, "hkv_decode_attn: workspace %zu bytes, need %zu", ws_bytes, need);
     HKV_REQUIRE((((uintptr_t)wsp) & 255) == 0, HKV_ERR_ARG, "hkv_decode_attn: workspace must be 256-byte aligned");
 
@@ -1428,8 +1579,14 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     p.part_pair_stride = (int64_t)(pair_part_bytes(nrep, ms) / sizeof(float));
     p.nxcc = num_xcc();
     // one range per pair needs no hand-off (and must not leave a mask bit behind)
-    p.xcc_local = (BH % p.nxcc) == 0 && ms > 1 && !(a->flags & HKV_DECODE_AGENT_HANDOFF) ? 1 : 0;
+    // (shared-out ranges: the kv heads are innermost in the workgroup ids, not the pairs)
+    p.xcc_local = ((lin > 0 ? a->num_kv_heads : BH) % p.nxcc) == 0 && (ms > 1 || lin > 0) &&
+                          !(a->flags & HKV_DECODE_AGENT_HANDOFF)
+                      ? 1
+                      : 0;
     p.max_splits = ms;
+    p.lin_ranges = lin;
+    p.split_stride = split_stride_floats(nrep);
     {
         // slice merge: every range of a pair must be resident while it waits for the
         // others (one 8-wave workgroup per CU: the grid fits the CUs); a slice has at most
@@ -1441,8 +1598,9 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
         // path where ranges stop waiting and the last arrival merges every slice).
         const int nout = nrep * kHeadDim;
         const int S = (nout + ms - 1) / ms;
-        p.coop = (ms > 1 && (int64_t)BH * ms <= num_cus() && S <= 128 && ms < kArrivedMask) ? 1 : 0;
+        // Shared-out ranges decide per pair in the kernel.
         p.slice_outputs = S;
+        p.coop = (ms > 1 && (int64_t)BH * ms <= num_cus() && S <= 128 && ms < kArrivedMask) ? 1 : 0;
         const char* mw = getenv("HKV_DECODE_MERGE_WAIT_TICKS");
         p.merge_wait = (mw && mw[0]) ? strtoull(mw, nullptr, 10) : kMergeWaitTicks;
     }
@@ -1456,7 +1614,7 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
         p.tl = tl_ptr[dev];
         const char* w = getenv("HKV_TIMELINE_WAITS");
         p.tl_waits = (w && w[0] == '1') ? 1 : 0;
-        g_timeline_waves = (int64_t)BH * ms * kWaves;
+        g_timeline_waves = (lin > 0 ? (int64_t)a->num_kv_heads * lin : (int64_t)BH * ms) * kWaves;
     }
 #endif
     p.scores = a->scores;
@@ -1473,26 +1631,17 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     const size_t lds = lds_bytes(nrep);
     const bool det = (a->flags & HKV_DECODE_DETERMINISTIC) != 0;
     const bool sc = a->scores != nullptr;
-    const int var = (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0);
-#define HKV_DECODE_FN(v) decode_attn_kernel<((v) & 1) != 0, ((v) & 2) != 0, ((v) & 4) != 0>
-    static const void* const fns[8] = {(const void*)HKV_DECODE_FN(0), (const void*)HKV_DECODE_FN(1),
-                                       (const void*)HKV_DECODE_FN(2), (const void*)HKV_DECODE_FN(3),
-                                       (const void*)HKV_DECODE_FN(4), (const void*)HKV_DECODE_FN(5),
-                                       (const void*)HKV_DECODE_FN(6), (const void*)HKV_DECODE_FN(7)};
-    static std::atomic<uint64_t> raised[8];   // the merge area plus the static id window can exceed 64 KB
-    HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
-    const dim3 grid((unsigned)(BH * ms)), block(kThreads);
-    switch (var) {
-        case 0: hipLaunchKernelGGL((HKV_DECODE_FN(0)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 1: hipLaunchKernelGGL((HKV_DECODE_FN(1)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 2: hipLaunchKernelGGL((HKV_DECODE_FN(2)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 3: hipLaunchKernelGGL((HKV_DECODE_FN(3)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 4: hipLaunchKernelGGL((HKV_DECODE_FN(4)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 5: hipLaunchKernelGGL((HKV_DECODE_FN(5)), grid, block, lds, (hipStream_t)stream, p); break;
-        case 6: hipLaunchKernelGGL((HKV_DECODE_FN(6)), grid, block, lds, (hipStream_t)stream, p); break;
-        default: hipLaunchKernelGGL((HKV_DECODE_FN(7)), grid, block, lds, (hipStream_t)stream, p); break;
-    }
+    const int var = (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0) + (lin > 0 ? 8 : 0);
+#define HKV_DECODE_FN(v) decode_attn_kernel<((v) & 1) != 0, ((v) & 2) != 0, ((v) & 4) != 0, ((v) & 8) != 0>
+    static void (*const fns[16])(DecodeParams) = {
+        HKV_DECODE_FN(0),  HKV_DECODE_FN(1),  HKV_DECODE_FN(2),  HKV_DECODE_FN(3),  HKV_DECODE_FN(4),  HKV_DECODE_FN(5),
+        HKV_DECODE_FN(6),  HKV_DECODE_FN(7),  HKV_DECODE_FN(8),  HKV_DECODE_FN(9),  HKV_DECODE_FN(10), HKV_DECODE_FN(11),
+        HKV_DECODE_FN(12), HKV_DECODE_FN(13), HKV_DECODE_FN(14), HKV_DECODE_FN(15)};
 #undef HKV_DECODE_FN
+    static std::atomic<uint64_t> raised[16];   // the merge area plus the static id window can exceed 64 KB
+    HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
+    const dim3 grid((unsigned)(lin > 0 ? (int64_t)a->num_kv_heads * lin : BH * ms)), block(kThreads);
+    hipLaunchKernelGGL(fns[var], grid, block, lds, (hipStream_t)stream, p);
     HKV_LAUNCH_CHECK("decode_attn_kernel");
     return HKV_OK;
 }

@@ -358,3 +358,45 @@ def test_bad_block_id_sets_flag():
     c.bt[0, 1] = 10 ** 6
     c.run(workspace=ws)
     assert ws.error_flag() == 1
+
+
+@pytest.mark.parametrize("hq,hkv,splits", [(1, 1, 5), (8, 8, 32), (32, 8, 16), (28, 4, 27), (28, 4, 28), (28, 4, 64),
+                                           (16, 1, 63), (16, 1, 33), (32, 8, 17)])
+def test_slice_merge_lanes(hq, hkv, splits):
+    """The two lane counts of the slice merge (4 per output up to 32 ranges, then 16) at range
+    counts around the line, ranges without work among them."""
+    print("case: slice merge %d/%d splits %d" % (hq, hkv, splits), flush=True)
+    _check(Case(300 + splits, 1, hq, hkv, 16, [700], [90]), splits=splits)
+
+
+@pytest.mark.parametrize("B,hq,hkv,mid,recent", [
+    (1, 8, 2, 0, 192), (1, 8, 2, 0, 193),        # the last size in one range, the first in several
+    (3, 28, 4, 40, 100), (3, 14, 2, 1000, 16),   # pairs that do not divide the CUs
+    (5, 32, 8, 600, 400), (16, 32, 8, 100, 300),
+])
+def test_range_rule(B, hq, hkv, mid, recent):
+    """The library's own range count at its edges, against the oracle."""
+    from heterokv import ops
+    print("case: range rule B=%d %d/%d mid %d recent %d" % (B, hq, hkv, mid, recent), flush=True)
+    mids = [max(0, mid - 37 * b) for b in range(B)]
+    ws = ops.DecodeWorkspace(DEV)
+    _check(Case(400 + B, B, hq, hkv, 64, mids, [recent] * B), workspace=ws)
+    assert ws.error_flag() == 0
+
+
+@pytest.mark.parametrize("hq,hkv,mids,recents", [
+    (32, 8, [20000, 0, 40, 9000], [100, 0, 300, 17]),     # a sequence without a key but its sink, short and long
+    (28, 4, [70000, 100, 2500], [64, 500, 1]),            # kv heads not a multiple of the XCDs, 64 ranges a pair
+    (16, 2, [30000] * 5, [33, 200, 1, 90, 64]),           # one length, given per sequence
+    (8, 8, [400 + 100 * i for i in range(31)], [20] * 31),   # nearly as many sequences as ranges per head
+    (4, 1, [15000 * (i % 30 == 7) + 5 * i for i in range(64)], [10 + i for i in range(64)]),
+])
+def test_ranges_shared_by_length(hq, hkv, mids, recents):
+    """Ragged batches, whose ranges are shared out by length, against the oracle, twice on one
+    workspace (the hand-off words come back to rest), then with the device-scope hand-off."""
+    from heterokv import ops
+    print("case: shared ranges %d/%d B=%d" % (hq, hkv, len(mids)), flush=True)
+    c = Case(500 + len(mids), len(mids), hq, hkv, 16, mids, recents)
+    for ws in (ops.DecodeWorkspace(DEV), ops.DecodeWorkspace(DEV, agent_handoff=True)):
+        _check(c, workspace=ws)
+        assert ws.error_flag() == 0
