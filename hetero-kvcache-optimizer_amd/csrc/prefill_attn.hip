@@ -16,6 +16,7 @@
 #include "prefill_stage.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace hkv {
 namespace {
@@ -29,7 +30,7 @@ template <int kKind>
 __device__ __forceinline__ void finish(const PrefillParams& p, const TileMap& tm, int bh, int rb, int s, int tid,
                                        pf16v (&acc)[4], float m, float l) {
     const int hh = (tid >> 5) & 1, r0 = (tid >> 6) * kPfQ + (tid & 31);   // row of the unit
-    const int row = rb * kUnitRows + r0;
+    const int row = unit_row(p, rb, r0);
     if (row >= p.Sq * p.nrep) return;
     const int64_t own_row = (int64_t)bh * (p.Sq * p.nrep) + row;   // kFinishSerial
     if (p.finish == kFinishPieces || (kKind == kKindF16 && p.finish == kFinishSerial && tm.n4 > 0)) {
@@ -78,14 +79,14 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     const int BH = p.B * p.Hkv;
     // Dispatch goes round-robin over the 8 XCDs by workgroup id: with the pairs innermost,
     // the workgroups of one pair run on one XCD and share its L2 when the pairs are a
-    // multiple of 8.  The last units, with the most chunk tiles, come first.
+    // multiple of 8.  The first units, with the most chunk tiles, come first.
     const int bh = wg % BH;
-    const int rb = p.units - 1 - wg / BH % p.units;
+    const int rb = wg / BH % p.units;
     const int s = wg / BH / p.units, ns = p.pieces[kKind];
     const int b = bh / p.Hkv, h = bh - b * p.Hkv;
-    const int row0 = rb * kUnitRows + wave * kPfQ;
+    const int row0 = unit_row(p, rb, wave * kPfQ);   // this wave's first row
     TileMap tm;
-    make_tile_map(p, b, (rb * kUnitRows + kUnitRows - 1) / p.nrep + 1, tm);
+    make_tile_map(p, b, unit_last_row(p, rb) / p.nrep + 1, tm);
     const int tiles = kKind == kKindF16 ? tm.nf() : tm.n4;
     // both kinds, one after the other: the other kernel finishes a sequence without tiles
     // of this kind
@@ -94,6 +95,12 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     const int rounds = (tiles + kFlatBufs - 1) / kFlatBufs;
     const int t0 = rounds * s / ns * kFlatBufs, t1 = min(tiles, rounds * (s + 1) / ns * kFlatBufs);
     const int T = (t1 - t0 + kFlatBufs - 1) / kFlatBufs * kFlatBufs;
+    // of these, a wave attends those up to its last query's
+    int Tc = row0 < p.Sq * p.nrep ? T : 0;
+    if (kKind == kKindF16 && tm.nc > 0 && Tc > 0) {
+        const int last = tm.nf() - tm.nc + min((row0 + kPfQ - 1) / p.nrep, p.Sq - 1) / kPfT;
+        Tc = min(T, max(0, last - t0 + kFlatBufs) / kFlatBufs * kFlatBufs);
+    }
 
     ph8 qf[8];
     const int qrow = min((row0 + n) / p.nrep, p.Sq - 1);
@@ -110,13 +117,13 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     if (T > 0) {
         if (team == 0) {
             Stage<kKind, 0> pol(p, tm, fw, t0, t1);
-            flat_tiles(pol, tm, fw, lds, qf, acc, m, l, T);
+            flat_tiles(pol, tm, fw, lds, qf, acc, m, l, Tc, T);
         } else {
             // waves 4-7 (the V^T staging, the larger share of VALU work) win issue ties
             // against the older waves 0-3 on their SIMDs
             __builtin_amdgcn_s_setprio(1);
             Stage<kKind, 1> pol(p, tm, fw, t0, t1);
-            flat_tiles(pol, tm, fw, lds, qf, acc, m, l, T);
+            flat_tiles(pol, tm, fw, lds, qf, acc, m, l, Tc, T);
             __builtin_amdgcn_s_setprio(0);
         }
     }
@@ -128,13 +135,24 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     finish<kKind>(p, tm, bh, rb, s, tid, acc, m, l);
 }
 
-// One workgroup per CU: 8 waves (two per SIMD), up to 256 registers per wave.
+// One workgroup per CU: 8 waves (two per SIMD), up to 256 registers per wave.  kKinds: a bit
+// per kind of tiles in the grid.  A kernel for each set of kinds: with both kinds' loops in
+// every kernel, 12 registers spilled and 2048 queries over 131K INT4 keys took 4.37 ms, not
+// 4.27 (same box).
+template <int kKinds>
 __global__ __launch_bounds__(kFlatThreads, 1) void prefill_attn_kernel(PrefillParams p) {
     touch_kernel_args(p);
     extern __shared__ __align__(16) uint8_t lds_raw[];
-    const int n4 = p.B * p.Hkv * p.units * p.pieces[kKindInt4];
-    if ((int)blockIdx.x < n4) attend<kKindInt4>(p, blockIdx.x, lds_raw);
-    else attend<kKindF16>(p, (int)blockIdx.x - n4, lds_raw);
+    constexpr int kF16 = 1 << kKindF16, kInt4 = 1 << kKindInt4;
+    if constexpr (kKinds == kF16) {
+        attend<kKindF16>(p, blockIdx.x, lds_raw);
+    } else if constexpr (kKinds == kInt4) {
+        attend<kKindInt4>(p, blockIdx.x, lds_raw);
+    } else {
+        const int n4 = p.B * p.Hkv * p.units * p.pieces[kKindInt4];
+        if ((int)blockIdx.x < n4) attend<kKindInt4>(p, blockIdx.x, lds_raw);
+        else attend<kKindF16>(p, (int)blockIdx.x - n4, lds_raw);
+    }
 }
 
 // Merges the states of a unit's pieces (kFinishPieces).  One workgroup per 32 rows of
@@ -169,7 +187,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
         }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int row = rb * kUnitRows + sub + 8 * r;
+        const int row = unit_row(p, rb, sub + 8 * r);
         if (row >= p.Sq * p.nrep) continue;
         uint16_t* op = p.out + (int64_t)b * p.o_sb + (int64_t)(h * p.nrep + row % p.nrep) * p.o_sh +
                        (int64_t)(row / p.nrep) * p.o_st;
@@ -190,11 +208,12 @@ int num_cus() {
 }
 
 // Why split: 203 queries of 32/8 heads are 32 units on 256 CUs; over 32,960 keys they took
-// 945 us unsplit and 173 us in 8 pieces each (7 INT4, 1 fp16).  Why not always: every piece
+// 945 us unsplit and 155 us in 8 pieces each (7 INT4, 1 fp16).  Why not always: every piece
 // writes and reads 135 KB of states, 16 us for 256 pieces; 256 equal units gain nothing.
+// Pieces hold whole rounds of the loop (64 pieces for 18 tiles cost 98 us, 6 pieces 32 us).
 // What the schedules cost, in INT4 tiles of one workgroup (~2 us each).  Workgroups run
 // longest first, one per CU, so CU round k ends with workgroup k x CUs of that order.
-constexpr double kF16Tile = 1.1;       // an fp16 tile (4x the K/V bytes of an INT4 one)
+constexpr double kF16Tile = 1.03;      // an fp16 tile (4x the K/V bytes of an INT4 one)
 constexpr double kSegTiles = 1.5;      // pipeline start and end of one tile loop
 constexpr double kLaunchTiles = 2.0;   // one more launch in the stream
 constexpr double kPieceTiles = 0.03;   // one piece's states: 135 KB written and read at ~4 TB/s
@@ -205,18 +224,10 @@ struct Plan {
     int64_t state_rows;
 };
 
-// Time of `n` INT4 workgroups of `len` tiles each beside the fp16 ones: of every unit rb's
-// `pieces` pieces, with tiles + rb * step tiles per unit.
-double grid_tiles(int cus, int64_t bh, int units, int p4, double len4, int pf, double tiles_f, double step) {
-    const int64_t n4 = bh * units * p4, nf = bh * units * pf;
-    const double top = pf ? (tiles_f + step * units) / pf : 0;
+// Time of `n4` INT4 workgroups of len4 tiles each beside `nf` fp16 ones of lenf tiles.
+double grid_tiles(int cus, int64_t n4, double len4, int64_t nf, double lenf) {
     double t = 0;
-    for (int64_t r = 0; r < n4 + nf; r += cus) {
-        // the kind with the longer pieces first; fp16 pieces shorten with the unit
-        const int64_t i = len4 >= top ? r - n4 : r;
-        const bool f = len4 >= top ? r >= n4 : r < nf;
-        t += kSegTiles + (f ? (tiles_f + step * (units - (double)(i / (bh * pf)))) / pf : len4);
-    }
+    for (int64_t r = 0; r < n4 + nf; r += cus) t += kSegTiles + ((len4 >= lenf) == (r < (len4 >= lenf ? n4 : nf)) ? len4 : lenf);
     return t;
 }
 
@@ -228,8 +239,9 @@ Plan make_plan(int64_t bh, int nrep, int sq, const int64_t (&tiles)[2], bool chu
     const int64_t all = bh * best.units;
     const int cus = num_cus();
     const bool has4 = tiles[kKindInt4] > 0, hasf = tiles[kKindF16] > 0 || chunk || !has4, both = has4 && hasf;
-    const double len4 = (double)tiles[kKindInt4], lenf = (double)tiles[kKindF16] * kF16Tile;
-    const double step = chunk ? (double)(kUnitRows / kPfT) / nrep * kF16Tile : 0;
+    // the pairing of the rows evens out the chunk's tiles: about the middle row's per unit
+    const double len4 = (double)tiles[kKindInt4];
+    const double lenf = ((double)tiles[kKindF16] + (chunk ? 0.55 * sq / kPfT + 1 : 0)) * kF16Tile;
     best.pieces[kKindF16] = hasf;
     best.pieces[kKindInt4] = has4;
     best.finish = both ? kFinishSerial : kFinishOut;
@@ -237,25 +249,23 @@ Plan make_plan(int64_t bh, int nrep, int sq, const int64_t (&tiles)[2], bool chu
     // Many units per CU even out by themselves, and their states would take gigabytes.
     if (all > 2 * cus) return best;
     double t_best = both ? kLaunchTiles : 0;
-    if (has4) t_best += grid_tiles(cus, bh, best.units, 1, len4, 0, 0, 0);
-    if (hasf) t_best += grid_tiles(cus, bh, best.units, 0, 0, 1, lenf, step);
-    const double avgf = hasf ? lenf + step * (best.units + 1) / 2 : 0;
-    for (int rounds = 1; rounds <= 3; ++rounds) {
-        const int per_unit = (int)std::min<int64_t>(kMaxPieces, (int64_t)rounds * cus / all);
-        if (per_unit < 2) continue;
-        const int mid = both ? (int)(per_unit * len4 / (len4 + avgf) + 0.5) : has4 ? per_unit : 0;
-        for (int p4 = mid - 1; p4 <= mid + 1; ++p4) {
-            const int pf = per_unit - p4;
-            if (p4 < 0 || pf < 0 || (p4 > 0) != has4 || (pf > 0) != hasf) continue;
-            const double t = grid_tiles(cus, bh, best.units, p4, p4 ? len4 / p4 : 0, pf, lenf, step) + kLaunchTiles +
-                             (double)(all * per_unit) * kPieceTiles;
-            if (t < t_best && all * per_unit * kUnitRows <= max_rows) {
-                t_best = t;
-                best.finish = kFinishPieces;
-                best.pieces[kKindInt4] = p4;
-                best.pieces[kKindF16] = pf;
-                best.state_rows = all * per_unit * kUnitRows;
-            }
+    if (has4) t_best += grid_tiles(cus, all, std::ceil(len4 / kFlatBufs) * kFlatBufs, 0, 0);
+    if (hasf) t_best += grid_tiles(cus, 0, 0, all, lenf);
+    // pieces of up to `len` tiles of either kind, in the loop's rounds
+    for (int len = kFlatBufs; len <= 1024; len += std::max(kFlatBufs, len / 64 * kFlatBufs)) {
+        const auto pieces = [&](double tiles_k) { return (int)std::min<double>(kMaxPieces, std::ceil(tiles_k / len)); };
+        const int p4 = has4 ? pieces(len4) : 0, pf = hasf ? pieces(lenf) : 0;
+        const int64_t n = all * (p4 + pf);
+        if (p4 + pf < 2 || n * kUnitRows > max_rows) continue;
+        const auto longest = [](double tiles_k, int np) { return np ? std::ceil(std::ceil(tiles_k / kFlatBufs) / np) * kFlatBufs : 0; };
+        const double t = grid_tiles(cus, all * p4, longest(len4, p4), all * pf, longest(lenf, pf)) + kLaunchTiles +
+                         (double)n * kPieceTiles;
+        if (t < t_best) {
+            t_best = t;
+            best.finish = kFinishPieces;
+            best.pieces[kKindInt4] = p4;
+            best.pieces[kKindF16] = pf;
+            best.state_rows = n * kUnitRows;
         }
     }
     return best;
@@ -275,15 +285,21 @@ size_t chunk_ws_bytes(const HkvPrefillArgs* a) {
 }
 
 int launch_attn(PrefillParams& p, const Plan& pl, hipStream_t stream) {
-    static std::atomic<uint64_t> raised{0};   // four tile buffers exceed the 64 KB default
-    HKV_RAISE_LDS(prefill_attn_kernel, kFlatLdsBytes, raised);
+    static void (*const fns[4])(PrefillParams) = {nullptr, prefill_attn_kernel<1>, prefill_attn_kernel<2>,
+                                                  prefill_attn_kernel<3>};
+    static std::atomic<uint64_t> raised[4];   // four tile buffers exceed the 64 KB default
     p.units = pl.units;
     p.finish = pl.finish;
     const unsigned all = (unsigned)(p.B * p.Hkv * p.units);
     const bool serial = pl.finish == kFinishSerial;
     for (int kind = 0; kind < (serial ? 2 : 1); ++kind) {
-        for (int k = 0; k < 2; ++k) p.pieces[k] = serial && k != kind ? 0 : pl.pieces[k];
-        hipLaunchKernelGGL(prefill_attn_kernel, dim3(all * (unsigned)(p.pieces[0] + p.pieces[1])), dim3(kFlatThreads),
+        int kinds = 0;
+        for (int k = 0; k < 2; ++k) {
+            p.pieces[k] = serial && k != kind ? 0 : pl.pieces[k];
+            if (p.pieces[k] > 0) kinds |= 1 << k;
+        }
+        HKV_RAISE_LDS(fns[kinds], kFlatLdsBytes, raised[kinds]);
+        hipLaunchKernelGGL(fns[kinds], dim3(all * (unsigned)(p.pieces[0] + p.pieces[1])), dim3(kFlatThreads),
                            kFlatLdsBytes, stream, p);
         HKV_LAUNCH_CHECK("prefill_attn_kernel");
     }

@@ -3,11 +3,18 @@
 //
 // Rows.  The n_rep query heads of a GQA group share their kv head's keys, so a (sequence,
 // kv head) pair is one attention problem of Sq x n_rep rows; row r is query r / n_rep of
-// head r % n_rep.  A unit is kUnitRows consecutive rows, whatever n_rep: no wave sits on
+// head r % n_rep.  A unit is kUnitRows rows, whatever n_rep: no wave sits on
 // an absent head (with one wave per head, n_rep = 1 left three of four waves idle and
 // n_rep = 7 one of eight: 512 queries of 32 heads over 4096 keys each, 158 -> 90 us with
 // the repacking of the keys; 2048 queries of 28/4 heads over 4160 keys and themselves, 239
 // -> 204 us).
+//
+// A unit pairs the u-th half-unit of 128 consecutive rows with the u-th from the end:
+// waves 0-3 take the first, waves 4-7 the second, one of each on every SIMD.  With a causal
+// chunk the later half sees more of it, the earlier half's waves stop computing early, and
+// the others have the SIMD to themselves: the units' times differ less than with units of
+// consecutive rows, which took from 66 to 97 tiles' time on the 28/4-head chunk above (204 ->
+// 192 us; a tile attended by four waves takes ~0.8 of one attended by all eight).
 //
 // Work.  A unit's keys are tiles of 64 tokens of two kinds, each with its own staging: fp16
 // (the zones' tiles, then the chunk's up to the unit's last query) and INT4.  A piece is
@@ -80,6 +87,21 @@ struct PrefillParams {
     int pieces[2];               // per unit, by kind (0: the launch has no tiles of the kind)
     float* state;                // state rows [.][kStateFloats]
 };
+
+// The global row of row r (< kUnitRows) of unit rb: the halves of the pairing above.  A
+// middle half-unit paired with itself counts once: its second copy lies past every row.
+__device__ __forceinline__ int unit_row(const PrefillParams& p, int rb, int r) {
+    constexpr int kHalf = kUnitRows / 2;
+    const int halves = (p.Sq * p.nrep + kHalf - 1) / kHalf;
+    if (r < kHalf) return rb * kHalf + r;
+    return halves - 1 - rb == rb ? halves * kHalf : (halves - 1 - rb) * kHalf + (r - kHalf);
+}
+// The unit's last row.
+__device__ __forceinline__ int unit_last_row(const PrefillParams& p, int rb) {
+    constexpr int kHalf = kUnitRows / 2;
+    const int halves = (p.Sq * p.nrep + kHalf - 1) / kHalf;
+    return min((halves - rb) * kHalf, p.Sq * p.nrep) - 1;
+}
 
 // First state row of piece s of kind `kind` of unit `unit` (counted over all pairs).
 __device__ __forceinline__ int64_t piece_row(const PrefillParams& p, int kind, int unit, int s) {

@@ -175,7 +175,8 @@ __device__ __forceinline__ void pv_flat(const uint8_t* vt, int n, int hh, const 
     }
 }
 
-// The tile loop over tiles 0 .. T-1 (T a multiple of kFlatBufs).  The staging policy
+// The tile loop over tiles 0 .. T-1, of which this wave attends the first Tc (multiples of
+// kFlatBufs).  The staging policy
 // `pol` provides
 //   kRing                      register slots of staged records in flight
 //   start(tm, lds)             loads and stages tiles 0 and 1, fills the slots
@@ -187,7 +188,7 @@ __device__ __forceinline__ void pv_flat(const uint8_t* vt, int n, int hh, const 
 // and (m, l, acc) carry the online softmax of this wave's rows in and out.
 template <class Pol>
 __device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const FlatWave& w, uint8_t* lds, const ph8 (&qf)[8],
-                                           pf16v (&acc)[4], float& m, float& l, int T) {
+                                           pf16v (&acc)[4], float& m, float& l, int Tc, int T) {
     pol.start(tm, lds);
     flat_barrier();
     pf16v Sx[2][2];
@@ -201,7 +202,7 @@ __device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const Fl
     qk_begin(flat_buf(lds, 0), w.n, w.hh, a0, a1, Sx[0], -msafe);
     qk_steps<0, 8>(flat_buf(lds, 0), w.n, w.hh, qf, a0, a1, Sx[0]);
     __builtin_amdgcn_sched_barrier(0);
-    for (int t0 = 0; t0 < T; t0 += kFlatBufs) {
+    for (int t0 = 0; t0 < Tc; t0 += kFlatBufs) {
 #pragma unroll
         for (int uu = 0; uu < kFlatBufs; ++uu) {
             const int t = t0 + uu;
@@ -257,6 +258,16 @@ __device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const Fl
             }
             __builtin_amdgcn_sched_barrier(0);
             pol.refill(tm, uu % Pol::kRing, t + 2);
+            flat_barrier();
+        }
+    }
+    // Past this wave's last query (or without a row): it only stages its share for the others.
+    for (int t0 = Tc; t0 < T; t0 += kFlatBufs) {
+#pragma unroll
+        for (int uu = 0; uu < kFlatBufs; ++uu) {
+            const int x = t0 + uu + 2;
+            pol.stage(uu % Pol::kRing, flat_buf(lds, (uu + 2) % kFlatBufs), flat_bias(lds, (uu + 2) % kFlatBufs), x);
+            pol.refill(tm, uu % Pol::kRing, x);
             flat_barrier();
         }
     }

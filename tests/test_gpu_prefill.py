@@ -286,3 +286,12 @@ def test_split_matches_unsplit(hq, hkv, sq, io):
     torch.cuda.synchronize()
     pool.check_errors()
     assert (a - b).abs().max().item() <= 2 * (2.0 ** -10 if io == torch.float16 else 2.0 ** -7)
+
+
+@pytest.mark.parametrize("hq,hkv,sq,recent", [(2, 2, 127, 0), (2, 2, 128, 70), (2, 2, 129, 0), (2, 2, 257, 64),
+                                              (1, 1, 385, 10), (14, 2, 55, 0), (7, 1, 110, 300), (3, 1, 43, 1)])
+def test_paired_half_units(hq, hkv, sq, recent):
+    """Row counts around the half-units of 128 rows that a unit pairs (a middle one without a
+    partner, a last one of one row), whose waves stop at different chunk tiles."""
+    print("case: paired half-units %d/%d Sq=%d recent %d" % (hq, hkv, sq, recent), flush=True)
+    _case(80 + sq, 1, hq, hkv, sq, 0, [0], [recent])
