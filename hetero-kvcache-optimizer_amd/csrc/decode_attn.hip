@@ -127,6 +127,7 @@ constexpr int kTlWords = 16;
 // Bytes one kv head reads per item (the weights that balance the ranges).
 constexpr int64_t kInt4ItemBytes = kBlockTokens * (kHeadDim / 2 + 5) * 2;   // 2208
 constexpr int64_t kF16ItemBytes = kBlockTokens * kHeadDim * 2 * 2;           // 8192
+constexpr int64_t kRefItemBytes = kBlockTokens * (kHeadDim + 5) * 2;         // 4256: unpacked codes
 // Balance weight of an INT4 block against an fp16 tile (8192): its 2208 bytes plus the
 // block-id indirection (INT4-only ranges start streaming only when their first ids are in
 // LDS, ~2.5 us into the 32K decode) and the nibble decode; fitted on the 32K decode,
@@ -143,6 +144,14 @@ struct ZoneP {
     int cap;
     int max_len;
     const int32_t* lens;
+};
+
+// INT4 keys and values in the unpacked reference layout (kRef): one byte per code,
+// [batch][kv head][len][128], with a float scale and a byte zero point per row.
+struct RefSource {
+    const uint8_t *kc, *vc;
+    const float *ks, *vs;
+    const uint8_t *kz, *vz;
 };
 
 struct DecodeParams {
@@ -162,6 +171,7 @@ struct DecodeParams {
     int bt_stride;
     const int32_t* int4_lens;
     int int4_max_len;
+    RefSource ref;
     uint16_t* out;
     int64_t o_sb, o_sh;
     int* err;
@@ -532,6 +542,108 @@ __device__ __forceinline__ void step_int4_pair(const Int4Blk& A, const Int4Blk& 
     }
 }
 
+// One 16-token block of the unpacked reference layout, attended in place: reading the codes
+// once, twice the packed bytes, instead of clearing a pool, repacking into it and reading
+// that (16384 tokens x 32 heads, 140 MB: 107 -> 36 us a call).  Lane (c, g) holds K row c's codes of
+// dims 32g .. 32g + 31 and, of the rows of tokens 4g .. 4g + 3, V codes of dims 8c .. 8c + 7
+// (so MFMA n of P.V takes dim 8c + n where the pool's layout gives c + 16n).
+struct RefBlk {
+    u4 k[2];
+    u2 v[4];
+    float ks[4], vs[4];   // of tokens 4g .. 4g + 3
+    uint32_t kz;          // of token c
+    uint32_t vz;          // of tokens 4g .. 4g + 3 (bytes)
+};
+// kVec: rows of a multiple of 4 tokens, whose scales and zero points load as vectors.  The
+// resources end with the block's valid rows: what lies past them reads as zero.
+template <bool kVec>
+__device__ __forceinline__ void load_ref(const DecodeParams& p, int64_t bh, int blk, bool valid, int c, int g, RefBlk& d) {
+    const int64_t row = bh * p.int4_max_len + (int64_t)blk * kBlockTokens;
+    const int n = valid ? min(kBlockTokens, p.int4_max_len - blk * kBlockTokens) : 0;
+    const __amdgpu_buffer_rsrc_t rk = rsrc(p.ref.kc + row * kHeadDim, n * kHeadDim);
+    const __amdgpu_buffer_rsrc_t rv = rsrc(p.ref.vc + row * kHeadDim, n * kHeadDim);
+    const __amdgpu_buffer_rsrc_t rks = rsrc(p.ref.ks + row, n * 4), rvs = rsrc(p.ref.vs + row, n * 4);
+    const __amdgpu_buffer_rsrc_t rkz = rsrc(p.ref.kz + row, n), rvz = rsrc(p.ref.vz + row, n);
+    d.k[0] = ld16(rk, c * kHeadDim + 32 * g);
+    d.k[1] = ld16(rk, c * kHeadDim + 32 * g + 16);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        d.v[t] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rv, (4 * g + t) * kHeadDim + 8 * c, 0, 0));
+    d.kz = __builtin_amdgcn_raw_buffer_load_b8(rkz, c, 0, 0);
+    if constexpr (kVec) {
+        const f4 a = __builtin_bit_cast(f4, ld16(rks, 16 * g)), b = __builtin_bit_cast(f4, ld16(rvs, 16 * g));
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            d.ks[t] = a[t];
+            d.vs[t] = b[t];
+        }
+        d.vz = ld4(rvz, 4 * g);
+    } else {
+        d.vz = 0u;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            d.ks[t] = __uint_as_float(ld4(rks, (4 * g + t) * 4));
+            d.vs[t] = __uint_as_float(ld4(rvs, (4 * g + t) * 4));
+            d.vz |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(rvz, 4 * g + t, 0, 0) << (8 * t);
+        }
+    }
+}
+// The four codes of a word as two exact fp16 pairs 1024 + code, minus 1024 + zp.  Only the
+// low four bits of a code count, as in the packed pool.
+__device__ __forceinline__ void ref_k_pairs(uint32_t w, h2 z, h2& lo, h2& hi) {
+    const uint32_t m = w & 0x0F0F0F0Fu;
+    lo = as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04010400u)) - z;
+    hi = as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04030402u)) - z;
+}
+// The two tokens' codes of byte e of their words, as an exact fp16 pair minus their zp.
+__device__ __forceinline__ h2 ref_v_pair(uint32_t w0, uint32_t w1, int e, h2 z) {
+    return as_h2(and_or(__builtin_amdgcn_perm(w1, w0, 0x0C000C00u | (uint32_t)e | ((uint32_t)(4 + e) << 16)),
+                        0x000F000Fu, 0x64006400u)) - z;
+}
+__device__ __forceinline__ void step_ref_pair(const RefBlk& A, const RefBlk& B, int nA, int nB, int g, const h8 (&qf)[4],
+                                              float scale_log2, f4 (&acc)[8], float& m, float& l) {
+    f4 SA = {0.f, 0.f, 0.f, 0.f}, SB = {0.f, 0.f, 0.f, 0.f};
+    const h2 zkA = zp1024(A.kz, A.kz), zkB = zp1024(B.kz, B.kz);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        h2 a[4], b[4];
+        ref_k_pairs(A.k[j >> 1][2 * (j & 1)], zkA, a[0], a[1]);
+        ref_k_pairs(A.k[j >> 1][2 * (j & 1) + 1], zkA, a[2], a[3]);
+        ref_k_pairs(B.k[j >> 1][2 * (j & 1)], zkB, b[0], b[1]);
+        ref_k_pairs(B.k[j >> 1][2 * (j & 1) + 1], zkB, b[2], b[3]);
+        SA = __builtin_amdgcn_mfma_f32_16x16x32_f16(h8{a[0][0], a[0][1], a[1][0], a[1][1], a[2][0], a[2][1], a[3][0], a[3][1]},
+                                                    qf[j], SA, 0, 0, 0);
+        SB = __builtin_amdgcn_mfma_f32_16x16x32_f16(h8{b[0][0], b[0][1], b[1][0], b[1][1], b[2][0], b[2][1], b[3][0], b[3][1]},
+                                                    qf[j], SB, 0, 0, 0);
+    }
+    const h2 zA01 = zp1024(A.vz & 0xffu, (A.vz >> 8) & 0xffu), zA23 = zp1024((A.vz >> 16) & 0xffu, A.vz >> 24);
+    const h2 zB01 = zp1024(B.vz & 0xffu, (B.vz >> 8) & 0xffu), zB23 = zp1024((B.vz >> 16) & 0xffu, B.vz >> 24);
+    h8 V[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+        const h2 a01 = ref_v_pair(A.v[0][n >> 2], A.v[1][n >> 2], n & 3, zA01);
+        const h2 a23 = ref_v_pair(A.v[2][n >> 2], A.v[3][n >> 2], n & 3, zA23);
+        const h2 b01 = ref_v_pair(B.v[0][n >> 2], B.v[1][n >> 2], n & 3, zB01);
+        const h2 b23 = ref_v_pair(B.v[2][n >> 2], B.v[3][n >> 2], n & 3, zB23);
+        V[n] = h8{a01[0], a01[1], a23[0], a23[1], b01[0], b01[1], b23[0], b23[1]};
+    }
+    float s[8], pr[8];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        s[v] = (4 * g + v < nA) ? SA[v] * (A.ks[v] * scale_log2) : -INFINITY;
+        s[4 + v] = (4 * g + v < nB) ? SB[v] * (B.ks[v] * scale_log2) : -INFINITY;
+    }
+    softmax_update<8>(s, acc, m, l, pr);
+    h8 P;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        P[v] = (_Float16)((4 * g + v < nA) ? pr[v] * A.vs[v] : 0.0f);
+        P[4 + v] = (_Float16)((4 * g + v < nB) ? pr[4 + v] * B.vs[v] : 0.0f);
+    }
+#pragma unroll
+    for (int n = 0; n < 8; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(V[n], P, acc[n], 0, 0, 0);
+}
+
 template <bool kScores = false>
 __device__ __forceinline__ void step_f16(F16Tile& d, int nvalid, int g, const h8 (&qf)[4],
                                          float scale_log2, f4 (&acc)[8], float& m, float& l, bool store = false,
@@ -746,8 +858,9 @@ __device__ __forceinline__ void load_partials(__amdgpu_buffer_rsrc_t prs, const 
 
 // kL2: the XCD-local hand-off (p.xcc_local), a template parameter so that each hand-off's
 // kernel carries only its own tail code.  kShared: p.lin_ranges > 0, for the same reason
-// (in one kernel with it, the 32K decode's launch was 0.25 us longer).
-template <bool kDynamic, bool kScores, bool kL2, bool kShared>
+// (in one kernel with it, the 32K decode's launch was 0.25 us longer).  kSrc: where the INT4 tokens are.
+enum : int { kSrcPool = 0, kSrcRef = 1, kSrcRefVec = 2 };   // unpacked layout; vector scales (load_ref)
+template <bool kDynamic, bool kScores, bool kL2, bool kShared, int kSrc = kSrcPool>
 __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     touch_kernel_args(p);   // the range plan below reads the arguments in a dependent chain
     int b, h, split, nsplit, first = 0;
@@ -817,7 +930,7 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     // The block ids of the first INT4 window are requested before anything else;
     // the fp16 tiles are streamed while they are on their way.
     int idr[kIdPerThread];
-    fetch_block_ids(p, b, a0, min(kIdWindow, a1 - a0), idr);
+    if constexpr (kSrc == kSrcPool) fetch_block_ids(p, b, a0, min(kIdWindow, a1 - a0), idr);
     __builtin_amdgcn_sched_barrier(0);
 
     // q fragments: lane (c, g) holds q[head c][32g + 8j .. +8] for step j.
@@ -865,7 +978,7 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     // every later slot is empty too.  An exit from inside the round would add a path
     // on which the later slots were not refilled, and the waits at the loop head
     // would then drain every slot.
-    if (nf > 0) {
+    if (kSrc == kSrcPool && nf > 0) {
         F16Tile buf[kF16Depth];
         int tq[kF16Depth];
         ZoneP zq[kF16Depth];
@@ -921,15 +1034,50 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
         }
     }
 
+    // ---- unpacked INT4 blocks a0 .. a1, two per step; every address follows from the block
+    // number, so the first loads need no ids
+    if constexpr (kSrc != kSrcPool) {
+        const int nblk = a1 - a0, npairs = (nblk + 1) >> 1;
+        RefBlk bufA[kPrefetch], bufB[kPrefetch];
+        int pk[kPrefetch];
+        int seq = wave + kPrefetch * kWaves;
+#pragma unroll
+        for (int k = 0; k < kPrefetch; ++k) {
+            pk[k] = wave + k * kWaves;
+            load_ref<kSrc == kSrcRefVec>(p, bh, a0 + 2 * pk[k], pk[k] < npairs, c, g, bufA[k]);
+            load_ref<kSrc == kSrcRefVec>(p, bh, a0 + 2 * pk[k] + 1, 2 * pk[k] + 1 < nblk, c, g, bufB[k]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();   // the counters
+        int nxt = next_unit<kDynamic>(&sm_ctr[0], seq);
+        if (pk[0] < npairs) {
+            do {
+#pragma unroll
+                for (int k = 0; k < kPrefetch; ++k) {
+                    const int lb = a0 + 2 * pk[k];
+                    const int nA = pk[k] < npairs ? min(kBlockTokens, len4 - lb * kBlockTokens) : 0;
+                    const int nB = (2 * pk[k] + 1 < nblk) ? min(kBlockTokens, len4 - (lb + 1) * kBlockTokens) : 0;
+                    step_ref_pair(bufA[k], bufB[k], nA, nB, g, qf, p.scale_log2, acc, m, l);
+                    pk[k] = nxt;
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_ref<kSrc == kSrcRefVec>(p, bh, a0 + 2 * nxt, nxt < npairs, c, g, bufA[k]);
+                    load_ref<kSrc == kSrcRefVec>(p, bh, a0 + 2 * nxt + 1, 2 * nxt + 1 < nblk, c, g, bufB[k]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    nxt = next_unit<kDynamic>(&sm_ctr[0], seq);
+                }
+            } while (pk[0] < npairs);
+        }
+    }
+
     // ---- INT4 blocks a0 .. a1, two per step, in windows of kIdWindow block ids
     // staged in LDS (same loop shape).  An empty slot re-reads the window's last
     // pair, an in-bounds address.
-    if (nf <= 0 && a1 > a0) {
+    if (kSrc == kSrcPool && nf <= 0 && a1 > a0) {
         commit_block_ids(p, min(kIdWindow, a1 - a0), idr, sm_ids);
         __syncthreads();
         TL_MARK(1);
     }
-    for (int wb = a0; wb < a1; wb += kIdWindow) {
+    for (int wb = a0; kSrc == kSrcPool && wb < a1; wb += kIdWindow) {
         const int wn = min(kIdWindow, a1 - wb);
         if (wb != a0) {
             fetch_block_ids(p, b, wb, wn, idr);
@@ -1032,7 +1180,7 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
 #pragma unroll
         for (int n = 0; n < 8; ++n)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) o[16 * n + 4 * g + v] = acc[n][v];
+            for (int v = 0; v < 4; ++v) o[kSrc == kSrcPool ? 16 * n + 4 * g + v : 8 * (4 * g + v) + n] = acc[n][v];
         if (g == 0) {
             sm_m[wave * 16 + c] = m;
             sm_l[wave * 16 + c] = l;
@@ -1363,8 +1511,8 @@ Ranges choose_ranges(int B, int Hkv, int nrep, int int4_max_len, int64_t int4_it
 
 // The fewest ranges a call without a hint may be cut to when its workspace is smaller than
 // the documented size: about one workgroup per CU, each reading at least ~96 KB.
-int least_splits(int BH, int int4_max_len, const int32_t* f16_max_lens, int nz) {
-    int64_t bytes = (int64_t)((int4_max_len + kBlockTokens - 1) / kBlockTokens) * kInt4ItemBytes;
+int least_splits(int BH, int int4_max_len, int64_t int4_item_bytes, const int32_t* f16_max_lens, int nz) {
+    int64_t bytes = (int64_t)((int4_max_len + kBlockTokens - 1) / kBlockTokens) * int4_item_bytes;
     for (int i = 0; i < nz; ++i) bytes += (int64_t)((f16_max_lens[i] + kBlockTokens - 1) / kBlockTokens) * kF16ItemBytes;
     int64_t s = (num_cus() + BH - 1) / BH;
     const int64_t by_size = (bytes + 96 * 1024 - 1) / (96 * 1024);
@@ -1458,9 +1606,10 @@ extern "C" int64_t hkv_decode_timeline_read(unsigned long long* host, int64_t ma
 }
 #endif
 
-// The launch behind both decode entry points: `wsp` / `ws_bytes` is the caller's
-// workspace (hkv_decode_attn) or this device's static scratch (hkv_decode_attn_noalloc).
-static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, void* stream) {
+// The launch behind the decode entry points: `wsp` / `ws_bytes` is the caller's workspace
+// (hkv_decode_attn, hkv_fused_decode) or this device's static scratch
+// (hkv_decode_attn_noalloc); `ref` is null, or holds the INT4 tokens in place of the pool.
+static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, void* stream, const RefSource* ref = nullptr) {
     HKV_REQUIRE(a->head_dim == kHeadDim, HKV_ERR_UNSUPPORTED, "hkv_decode_attn: head_dim %d != 128", a->head_dim);
     HKV_REQUIRE(a->batch > 0 && a->num_kv_heads > 0 && a->num_q_heads > 0, HKV_ERR_ARG,
                 "hkv_decode_attn: bad batch/heads");
@@ -1489,7 +1638,7 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
                 HKV_ERR_ARG, "hkv_decode_attn: q must be 16-byte aligned with strides multiple of 8");
     HKV_REQUIRE(a->int4_max_len >= 0 && a->int4_max_len <= kMaxZoneTokens, HKV_ERR_ARG,
                 "hkv_decode_attn: int4_max_len %d outside [0, %d]", a->int4_max_len, kMaxZoneTokens);
-    if (a->int4_max_len > 0) {
+    if (a->int4_max_len > 0 && !ref) {
         HKV_REQUIRE(a->block_table && ((a->pool && a->pool_blocks > 0) || (a->staging && a->staging_blocks > 0)),
                     HKV_ERR_ARG, "hkv_decode_attn: INT4 zone without pool/staging records or block table");
         HKV_REQUIRE(a->pool_blocks >= 0 && a->staging_blocks >= 0 && a->staging_blocks <= (1ll << 31),
@@ -1520,11 +1669,11 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     HKV_REQUIRE(BH < 65536, HKV_ERR_ARG, "hkv_decode_attn: batch x kv heads too large");
     bool own_lens = a->int4_lens != nullptr;
     for (int i = 0; i < a->num_f16_zones; ++i) own_lens = own_lens || a->f16[i].lens != nullptr;
-    const Ranges rg = choose_ranges(a->batch, a->num_kv_heads, nrep, a->int4_max_len, kInt4ItemBytes, zl,
+    const Ranges rg = choose_ranges(a->batch, a->num_kv_heads, nrep, a->int4_max_len, ref ? kRefItemBytes : kInt4ItemBytes, zl,
                                     a->num_f16_zones, own_lens, a->splits_hint);
     int ms = rg.per_pair, lin = rg.lin;
     if (a->splits_hint <= 0) {
-        const int least = least_splits((int)BH, a->int4_max_len, zl, a->num_f16_zones);
+        const int least = least_splits((int)BH, a->int4_max_len, ref ? kRefItemBytes : kInt4ItemBytes, zl, a->num_f16_zones);
         if (lin > 0 && shared_workspace_bytes(a->num_kv_heads, nrep, lin) > ws_bytes) {
             lin = 0;
             ms = least;
@@ -1567,6 +1716,7 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     p.bt_stride = a->bt_stride;
     p.int4_lens = a->int4_lens;
     p.int4_max_len = a->int4_max_len;
+    p.ref = ref ? *ref : RefSource{};
     p.out = a->out;
     p.o_sb = a->out_stride_b;
     p.o_sh = a->out_stride_h;
@@ -1631,14 +1781,20 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     const size_t lds = lds_bytes(nrep);
     const bool det = (a->flags & HKV_DECODE_DETERMINISTIC) != 0;
     const bool sc = a->scores != nullptr;
-    const int var = (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0) + (lin > 0 ? 8 : 0);
+    // pool: by schedule, scores, hand-off and range plan; unpacked layout (lengths of its own
+    // do not occur): by hand-off and row alignment
+    const int var = ref ? 16 + (p.xcc_local ? 1 : 0) + (a->int4_max_len % 4 == 0 ? 2 : 0)
+                        : (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0) + (lin > 0 ? 8 : 0);
 #define HKV_DECODE_FN(v) decode_attn_kernel<((v) & 1) != 0, ((v) & 2) != 0, ((v) & 4) != 0, ((v) & 8) != 0>
-    static void (*const fns[16])(DecodeParams) = {
-        HKV_DECODE_FN(0),  HKV_DECODE_FN(1),  HKV_DECODE_FN(2),  HKV_DECODE_FN(3),  HKV_DECODE_FN(4),  HKV_DECODE_FN(5),
-        HKV_DECODE_FN(6),  HKV_DECODE_FN(7),  HKV_DECODE_FN(8),  HKV_DECODE_FN(9),  HKV_DECODE_FN(10), HKV_DECODE_FN(11),
-        HKV_DECODE_FN(12), HKV_DECODE_FN(13), HKV_DECODE_FN(14), HKV_DECODE_FN(15)};
+#define HKV_DECODE_REF(v) decode_attn_kernel<true, false, ((v) & 1) != 0, false, ((v) & 2) != 0 ? kSrcRefVec : kSrcRef>
+    static void (*const fns[20])(DecodeParams) = {
+        HKV_DECODE_FN(0),  HKV_DECODE_FN(1),  HKV_DECODE_FN(2),  HKV_DECODE_FN(3),  HKV_DECODE_FN(4),
+        HKV_DECODE_FN(5),  HKV_DECODE_FN(6),  HKV_DECODE_FN(7),  HKV_DECODE_FN(8),  HKV_DECODE_FN(9),
+        HKV_DECODE_FN(10), HKV_DECODE_FN(11), HKV_DECODE_FN(12), HKV_DECODE_FN(13), HKV_DECODE_FN(14),
+        HKV_DECODE_FN(15), HKV_DECODE_REF(0), HKV_DECODE_REF(1), HKV_DECODE_REF(2), HKV_DECODE_REF(3)};
 #undef HKV_DECODE_FN
-    static std::atomic<uint64_t> raised[16];   // the merge area plus the static id window can exceed 64 KB
+#undef HKV_DECODE_REF
+    static std::atomic<uint64_t> raised[20];   // the merge area plus the static id window can exceed 64 KB
     HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
     const dim3 grid((unsigned)(lin > 0 ? (int64_t)a->num_kv_heads * lin : BH * ms)), block(kThreads);
     hipLaunchKernelGGL(fns[var], grid, block, lds, (hipStream_t)stream, p);
@@ -1650,6 +1806,35 @@ extern "C" int hkv_decode_attn(const HkvDecodeArgs* a, void* stream) {
     clear_error();
     HKV_REQUIRE(a != nullptr, HKV_ERR_ARG, "hkv_decode_attn: null args");
     return decode_launch(a, a->workspace, a->workspace_bytes, stream);
+}
+
+// ---- the reference's fused decode signature: attention straight from the unpacked codes
+extern "C" int hkv_fused_decode(const HkvFusedArgs* f, void* stream) {
+    clear_error();
+    HKV_REQUIRE(f != nullptr, HKV_ERR_ARG, "hkv_fused_decode: null args");
+    HKV_REQUIRE(f->num_queries == 1, HKV_ERR_ARG, "hkv_fused_decode: one query per sequence, got %d", f->num_queries);
+    HKV_REQUIRE(f->num_tokens >= 0, HKV_ERR_ARG, "hkv_fused_decode: num_tokens < 0");
+    const int rc = check_fused_source(f, "hkv_fused_decode");
+    if (rc != HKV_OK) return rc;
+    HkvDecodeArgs a = {};
+    a.batch = f->batch;
+    a.num_q_heads = f->num_q_heads;
+    a.num_kv_heads = f->num_kv_heads;
+    a.head_dim = f->head_dim;
+    a.sm_scale = f->sm_scale;
+    a.q = f->q;
+    a.q_stride_b = f->q_stride_b;
+    a.q_stride_h = f->q_stride_h;
+    a.int4_max_len = f->num_tokens;
+    a.out = f->out;
+    a.out_stride_b = f->out_stride_b;
+    a.out_stride_h = f->out_stride_h;
+    a.flags = f->flags;
+    a.q_dtype = f->q_dtype;
+    a.out_dtype = f->out_dtype;
+    a.err_flag = f->err_flag;
+    const RefSource ref = {f->k_codes, f->v_codes, f->k_scales, f->v_scales, f->k_zps, f->v_zps};
+    return decode_launch(&a, f->workspace, f->workspace_bytes, stream, &ref);
 }
 
 // ---- allocation-free variant: the partial states, tickets and XCD masks live in a

@@ -58,6 +58,18 @@ void clear_error();
         }                                                                                     \
     } while (0)
 
+// The unpacked INT4 source of the fused entry points: present and aligned for the kernels'
+// vector loads.
+inline int check_fused_source(const HkvFusedArgs* f, const char* name) {
+    if (f->num_tokens == 0) return HKV_OK;
+    HKV_REQUIRE(f->k_codes && f->v_codes && f->k_scales && f->v_scales && f->k_zps && f->v_zps, HKV_ERR_ARG,
+                "%s: null pointer", name);
+    HKV_REQUIRE((((uintptr_t)f->k_codes | (uintptr_t)f->v_codes | (uintptr_t)f->k_scales | (uintptr_t)f->v_scales) & 15) == 0 &&
+                    (((uintptr_t)f->k_zps | (uintptr_t)f->v_zps) & 3) == 0,
+                HKV_ERR_ARG, "%s: codes and scales must be 16-byte aligned, zero points 4-byte", name);
+    return HKV_OK;
+}
+
 constexpr int kHeadDim = 128;
 constexpr int kBlockTokens = 16;
 constexpr int kCodeRowBytes = kHeadDim / 2;          // 64 B of packed codes per token row

@@ -256,7 +256,7 @@ Plan make_plan(int64_t bh, int nrep, int sq, const int64_t (&tiles)[2], bool chu
         const auto pieces = [&](double tiles_k) { return (int)std::min<double>(kMaxPieces, std::ceil(tiles_k / len)); };
         const int p4 = has4 ? pieces(len4) : 0, pf = hasf ? pieces(lenf) : 0;
         const int64_t n = all * (p4 + pf);
-        if (p4 + pf < 2 || n * kUnitRows > max_rows) continue;
+        if (p4 + pf < 2 || n > 4 * cus || n * kUnitRows > max_rows) continue;
         const auto longest = [](double tiles_k, int np) { return np ? std::ceil(std::ceil(tiles_k / kFlatBufs) / np) * kFlatBufs : 0; };
         const double t = grid_tiles(cus, all * p4, longest(len4, p4), all * pf, longest(lenf, pf)) + kLaunchTiles +
                          (double)n * kPieceTiles;

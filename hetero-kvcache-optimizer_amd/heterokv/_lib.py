@@ -127,6 +127,16 @@ class PrefillArgs(ctypes.Structure):
                 ("workspace", vp), ("workspace_bytes", ctypes.c_size_t)]
 
 
+class FusedArgs(ctypes.Structure):
+    _fields_ = [("batch", i32), ("num_q_heads", i32), ("num_kv_heads", i32), ("head_dim", i32),
+                ("num_queries", i32), ("num_tokens", i32), ("sm_scale", ctypes.c_float),
+                ("q_dtype", i32), ("out_dtype", i32), ("flags", i32),
+                ("q", vp), ("q_stride_b", i64), ("q_stride_h", i64), ("q_stride_t", i64),
+                ("k_codes", vp), ("v_codes", vp), ("k_scales", vp), ("v_scales", vp), ("k_zps", vp), ("v_zps", vp),
+                ("out", vp), ("out_stride_b", i64), ("out_stride_h", i64), ("out_stride_t", i64),
+                ("err_flag", vp), ("workspace", vp), ("workspace_bytes", ctypes.c_size_t)]
+
+
 class CopyDesc(ctypes.Structure):
     _fields_ = [("dst", vp), ("src", vp), ("bytes", ctypes.c_size_t)]
 
@@ -157,6 +167,7 @@ SYMBOLS = [
     ("hkv_prefill_workspace_bytes", ctypes.c_size_t, [i32, i32, i32]),
     ("hkv_prefill_split_bytes", ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
     ("hkv_prefill_attn", ctypes.c_int, [ctypes.POINTER(PrefillArgs), vp]),
+    ("hkv_fused_decode", ctypes.c_int, [ctypes.POINTER(FusedArgs), vp]),
     ("hkv_pf_create", ctypes.c_int, [i32, ctypes.c_size_t, i32, ctypes.POINTER(vp)]),
     ("hkv_pf_destroy", ctypes.c_int, [vp]),
     ("hkv_pf_host_ptr", vp, [vp, ctypes.c_size_t]),

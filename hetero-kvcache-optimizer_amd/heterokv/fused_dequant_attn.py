@@ -10,9 +10,9 @@ sm_scale defaulting to 1/sqrt(head_dim).  Unlike the reference's Triton kernel
 exactly that formula, and it also accepts GQA (q heads a multiple of kv heads).
 
 The reference passes unpacked codes (one uint8 per value) with per-token
-scales/zps [B, H, S]; they are repacked into INT4 block records on the device
-(hkv_repack_codes) and attended by the split-K decode kernel (hkv_decode_attn) or the
-MFMA prefill kernel (hkv_prefill_attn).  q may be fp16 or bf16 (bf16 is narrowed to
+scales/zps [B, H, S].  Decode attends them as they are (hkv_fused_decode, the split-K
+decode kernel); forward repacks them into INT4 block records on the device
+(hkv_repack_codes) for the MFMA prefill kernel (hkv_prefill_attn).  q may be fp16 or bf16 (bf16 is narrowed to
 fp16 operands exactly within the fp16 range).  Device errors (an out-of-range bf16
 value, a decode placement failure) go to a per-device error word that is read without
 blocking at the next call -- a later call raises HeteroKVError -- or at once by
@@ -85,16 +85,10 @@ def fused_dequant_attn_decode(q: torch.Tensor, k_data: torch.Tensor, k_scales: t
     vz = v_zps.reshape(B, Hkv, S)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
-    nblk = (S + BLOCK_TOKENS - 1) // BLOCK_TOKENS
     err = _errword(q.device)
     err.poll()
-    pool = ops.Int4Pool(B * nblk, Hkv, q.device)
-    bt = torch.arange(B * nblk, dtype=torch.int32, device=q.device).reshape(B, nblk)
-    start = torch.zeros(B, dtype=torch.int32, device=q.device)
-    ops.repack_codes(pool, kd, vd, ks, vs, kz, vz, start, bt, err=err)
     qq = _as_kernel_q(q, err)
-    out = ops.decode_attention(qq, zones=(), pool=pool, block_table=bt, int4_lens=None, int4_max_len=S,
-                               sm_scale=sm_scale, workspace=_WS[q.device], err=err, out_dtype=qq.dtype)
+    out = ops.fused_decode(qq, kd, vd, ks, vs, kz, vz, sm_scale, _WS[q.device], err, qq.dtype)
     err.post()
     return out.to(q.dtype)
 

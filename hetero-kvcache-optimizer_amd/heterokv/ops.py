@@ -556,6 +556,50 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
     return out.unsqueeze(2) if squeeze else out
 
 
+# ----------------------------------------------------------------------- fused (unpacked INT4)
+def _row_tensor(t, shape, dtype):
+    """t as a contiguous `dtype` tensor of `shape` with a 16-byte aligned base."""
+    t = t.reshape(shape).to(dtype).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
+    """(FusedArgs, out, tensors to keep) of one call: q [B, Hq, Sq, 128], codes uint8
+    [B, Hkv, S, 128], scales / zps [B, Hkv, S]."""
+    _require_gpu(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps)
+    B, H, T, D = k_codes.shape
+    if D != HEAD_DIM or v_codes.shape != k_codes.shape:
+        raise HeteroKVError(-1, "fused attention: codes must be [B, H, T, 128]")
+    if q.dtype not in _F16_OR_BF16 or q.dim() != 4 or q.shape[-1] != HEAD_DIM or q.shape[0] != B:
+        raise HeteroKVError(-1, "fused attention: q must be fp16 or bf16 [B, Hq, Sq, 128]")
+    if q.stride(-1) != 1 or q.data_ptr() % 16 or any(st % 8 for st in q.stride()[:3]):
+        q = q.contiguous()
+    kc, vc = k_codes.contiguous(), v_codes.contiguous()
+    kc, vc = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (kc, vc))
+    ks, vs = (_row_tensor(t, (B, H, T), torch.float32) for t in (k_scales, v_scales))
+    # zero points as bytes; other types go through float32, the reference's type for them
+    kz, vz = (_row_tensor(t if t.dtype == k_zps.dtype == torch.uint8 else t.to(torch.float32), (B, H, T), torch.uint8)
+              for t in (k_zps, v_zps))
+    out = torch.empty(q.shape, dtype=out_dtype, device=q.device)
+    a = _lib.FusedArgs(batch=B, num_q_heads=q.shape[1], num_kv_heads=H, head_dim=HEAD_DIM, num_queries=q.shape[2],
+                       num_tokens=T, sm_scale=float(sm_scale), q_dtype=_DTYPES[q.dtype], out_dtype=_DTYPES[out_dtype],
+                       q=q.data_ptr(), q_stride_b=q.stride(0), q_stride_h=q.stride(1), q_stride_t=q.stride(2),
+                       k_codes=kc.data_ptr(), v_codes=vc.data_ptr(), k_scales=ks.data_ptr(), v_scales=vs.data_ptr(),
+                       k_zps=kz.data_ptr(), v_zps=vz.data_ptr(), out=out.data_ptr(), out_stride_b=out.stride(0),
+                       out_stride_h=out.stride(1), out_stride_t=out.stride(2), err_flag=err.ptr())
+    return a, out, (q, kc, vc, ks, vs, kz, vz)
+
+
+def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, workspace, err, out_dtype):
+    """hkv_fused_decode: decode attention (q [B, Hq, 1, 128]) straight from unpacked codes."""
+    a, out, keep = _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype)
+    ws = workspace.get(decode_workspace_bytes(a.batch, a.num_q_heads, a.num_kv_heads, a.num_tokens, ()))
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    a.flags = _lib.DECODE_AGENT_HANDOFF if workspace.agent_handoff else 0
+    check(load().hkv_fused_decode(ctypes.byref(a), stream_ptr(q.device)), "hkv_fused_decode")
+    return out
+
+
 # ----------------------------------------------------------------------- record gather
 def gather_blocks(src, ids, dst, staging=None, dst_offset=0, err=None):
     """dst record dst_offset + i = record ids[i] of src (ids >= 0) or of staging (~ids[i]).

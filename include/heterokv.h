@@ -417,6 +417,36 @@ size_t hkv_prefill_split_bytes(const HkvPrefillArgs* args);
 int hkv_prefill_attn(const HkvPrefillArgs* args, void* stream);
 
 /*
+ * The reference's fused kernels' own signature (kernels/fused_dequant_attn.py:301-368):
+ * decode attention of one query per sequence straight from unpacked codes, with the
+ * numerics of hkv_repack_codes + hkv_decode_attn (only the low four bits of a code count).
+ * codes: uint8 [batch][num_kv_heads][num_tokens][128], 16-byte aligned; scales: float and
+ * zps: uint8, [batch][num_kv_heads][num_tokens] (4-byte aligned zps where num_tokens is a
+ * multiple of 4).  Workspace, flags and error bits as in HkvDecodeArgs.
+ */
+typedef struct HkvFusedArgs {
+    int32_t batch, num_q_heads, num_kv_heads, head_dim, num_queries, num_tokens;
+    float sm_scale;
+    int32_t q_dtype, out_dtype;    /* F16 or BF16 */
+    int32_t flags;
+    const uint16_t* q;             /* [batch][num_q_heads][num_queries][128] with strides */
+    int64_t q_stride_b, q_stride_h, q_stride_t;
+    const uint8_t* k_codes;
+    const uint8_t* v_codes;
+    const float* k_scales;
+    const float* v_scales;
+    const uint8_t* k_zps;
+    const uint8_t* v_zps;
+    uint16_t* out;                 /* [batch][num_q_heads][num_queries][128] with strides */
+    int64_t out_stride_b, out_stride_h, out_stride_t;
+    int32_t* err_flag;
+    void* workspace;
+    size_t workspace_bytes;
+} HkvFusedArgs;
+
+int hkv_fused_decode(const HkvFusedArgs* args, void* stream);
+
+/*
  * Host-tier prefetcher (replaces DRAMStorageManager's per-tensor pinned dict,
  * dram_storage.py:106-194, and AsyncPrefetcher's side stream, prefetcher.py:33-111).
  * A handle owns a pinned host arena (hipHostMalloc), a side stream created at

@@ -295,3 +295,29 @@ def test_prefill_split_rule(lib):
     chunk = 2 * 8 * 64 * 128 * 2
     assert n > chunk and (n - chunk) % (8 * 256 * 132 * 4) == 0
     assert lib.hkv_prefill_split_bytes(None) == 0
+
+
+def test_fused_args(lib, tmp_path):
+    """HkvFusedArgs: gcc's layout, and the argument errors of the fused entry points."""
+    import shutil
+    import subprocess
+    from heterokv import _lib
+    a = _lib.FusedArgs(batch=1, num_q_heads=8, num_kv_heads=8, head_dim=128, num_queries=2, num_tokens=4)
+    _err(lib, lib.hkv_fused_decode(ctypes.byref(a), None), -1, b"one query")
+    a.num_queries = 1
+    _err(lib, lib.hkv_fused_decode(ctypes.byref(a), None), -1, b"null")
+    a.k_codes = a.v_codes = a.k_scales = a.v_scales = 4096
+    a.k_zps = a.v_zps = 4097
+    _err(lib, lib.hkv_fused_decode(ctypes.byref(a), None), -1, b"aligned")
+    a.k_zps = a.v_zps = 4096
+    a.head_dim = 64
+    _err(lib, lib.hkv_fused_decode(ctypes.byref(a), None), -4, b"head_dim")
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc not available")
+    src, exe = tmp_path / "fused.c", tmp_path / "fused"
+    src.write_text('#include <stdio.h>\n#include <stddef.h>\n#include "%s"\nint main(void){\n' % HEADER + "".join(
+        'printf("%%zu ", offsetof(HkvFusedArgs, %s));\n' % n for n, _ in _lib.FusedArgs._fields_) +
+        'printf("%zu", sizeof(HkvFusedArgs)); return 0;}')
+    subprocess.run(["gcc", "-o", str(exe), str(src)], check=True)
+    got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+    assert got == [getattr(_lib.FusedArgs, n).offset for n, _ in _lib.FusedArgs._fields_] + [ctypes.sizeof(_lib.FusedArgs)]
