@@ -22,7 +22,9 @@ namespace hkv {
 namespace {
 
 template <int kKind, int kTeam>
-using Stage = typename std::conditional<kKind == kKindF16, F16Stage<kTeam>, Int4Stage<kTeam>>::type;
+using Stage = typename std::conditional<
+    kKind == kKindF16, F16Stage<kTeam>,
+    typename std::conditional<kKind == kKindInt4, Int4Stage<kTeam>, RefStage<kTeam, kKind == kKindRefVec>>::type>::type;
 
 // Writes a piece's result: a state, or the output (with kFinishSerial, of the fp16
 // kernel's states and this one's).
@@ -32,12 +34,21 @@ __device__ __forceinline__ void finish(const PrefillParams& p, const TileMap& tm
     const int hh = (tid >> 5) & 1, r0 = (tid >> 6) * kPfQ + (tid & 31);   // row of the unit
     const int row = unit_row(p, rb, r0);
     if (row >= p.Sq * p.nrep) return;
+    const int wave = tid >> 6;
+    if (p.finish == kFinishPieces) {
+        float* st = piece_state(p, kKind, bh * p.units + rb, s);
+        pf4* o = (pf4*)st + (wave * 16) * 64 + (tid & 63);
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[(4 * db + j) * 64] = pf4{acc[db][4 * j + 0], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]};
+        if (hh == 0) *(float2*)(st + kPieceML + 2 * r0) = make_float2(m, l);
+        return;
+    }
     const int64_t own_row = (int64_t)bh * (p.Sq * p.nrep) + row;   // kFinishSerial
-    if (p.finish == kFinishPieces || (kKind == kKindF16 && p.finish == kFinishSerial && tm.n4 > 0)) {
-        const int64_t sr = p.finish == kFinishSerial
-                               ? own_row
-                               : piece_row(p, kKind, bh * p.units + rb, s) + r0;
-        float* st = p.state + sr * kStateFloats;
+    if (kKind == kKindF16 && p.finish == kFinishSerial && tm.n4 > 0) {
+        float* st = p.state + own_row * kStateFloats;
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -82,7 +93,8 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     // multiple of 8.  The first units, with the most chunk tiles, come first.
     const int bh = wg % BH;
     const int rb = wg / BH % p.units;
-    const int s = wg / BH / p.units, ns = p.pieces[kKind];
+    constexpr int kPlan = kKind == kKindF16 ? kKindF16 : kKindInt4;   // unpacked codes are INT4 tiles
+    const int s = wg / BH / p.units, ns = p.pieces[kPlan];
     const int b = bh / p.Hkv, h = bh - b * p.Hkv;
     const int row0 = unit_row(p, rb, wave * kPfQ);   // this wave's first row
     TileMap tm;
@@ -90,7 +102,7 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     const int tiles = kKind == kKindF16 ? tm.nf() : tm.n4;
     // both kinds, one after the other: the other kernel finishes a sequence without tiles
     // of this kind
-    if (p.finish == kFinishSerial && tiles == 0 && (kKind == kKindInt4 || tm.n4 > 0)) return;
+    if (p.finish == kFinishSerial && tiles == 0 && (kKind != kKindF16 || tm.n4 > 0)) return;
     // pieces start at multiples of the loop's round of kFlatBufs tiles
     const int rounds = (tiles + kFlatBufs - 1) / kFlatBufs;
     const int t0 = rounds * s / ns * kFlatBufs, t1 = min(tiles, rounds * (s + 1) / ns * kFlatBufs);
@@ -132,7 +144,7 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     // nothing of it lives in registers across the tile loop
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    finish<kKind>(p, tm, bh, rb, s, tid, acc, m, l);
+    finish<kPlan>(p, tm, bh, rb, s, tid, acc, m, l);
 }
 
 // One workgroup per CU: 8 waves (two per SIMD), up to 256 registers per wave.  kKinds: a bit
@@ -148,6 +160,10 @@ __global__ __launch_bounds__(kFlatThreads, 1) void prefill_attn_kernel(PrefillPa
         attend<kKindF16>(p, blockIdx.x, lds_raw);
     } else if constexpr (kKinds == kInt4) {
         attend<kKindInt4>(p, blockIdx.x, lds_raw);
+    } else if constexpr (kKinds == 1 << kKindRef) {
+        attend<kKindRef>(p, blockIdx.x, lds_raw);
+    } else if constexpr (kKinds == 1 << kKindRefVec) {
+        attend<kKindRefVec>(p, blockIdx.x, lds_raw);
     } else {
         const int n4 = p.B * p.Hkv * p.units * p.pieces[kKindInt4];
         if ((int)blockIdx.x < n4) attend<kKindInt4>(p, blockIdx.x, lds_raw);
@@ -155,44 +171,42 @@ __global__ __launch_bounds__(kFlatThreads, 1) void prefill_attn_kernel(PrefillPa
     }
 }
 
-// Merges the states of a unit's pieces (kFinishPieces).  One workgroup per 32 rows of
-// a unit, wave db over dims 32 db .. +31, 8 lanes per row.  Bound by the reads of the
-// states (528 B per row and piece), which the Infinity Cache mostly serves.
+// Merges the states of a unit's pieces (kFinishPieces).  One workgroup per 32 rows of a
+// unit (a wave's), wave db over dims 32 db .. +31, with the attention kernel's lane layout.
+// Bound by the reads of the states (520 B per row and piece), which the Infinity Cache
+// mostly serves: 256 pieces, 33 MB, in 7.8 us (11.7 us with row-major states, whose 16-byte
+// pieces of a wave's store lie in 32 rows).
 __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
     touch_kernel_args(p);
-    const int unit = (int)blockIdx.x >> 3;
+    const int unit = (int)blockIdx.x >> 3, wave = (int)blockIdx.x & 7;
     const int bh = unit / p.units, rb = unit - bh * p.units;
-    const int lane = threadIdx.x & 63, d = 32 * (threadIdx.x >> 6) + 4 * (lane & 7);
-    const int sub = ((int)blockIdx.x & 7) * kPfQ + (lane >> 3);   // rows sub + 8 i of the unit
+    const int lane = threadIdx.x & 63, db = threadIdx.x >> 6, n = lane & 31, hh = lane >> 5;
+    const int row = unit_row(p, rb, wave * kPfQ + n);
+    if (__ballot(row < p.Sq * p.nrep) == 0) return;
     const int np = p.pieces[0] + p.pieces[1];
-    const float* first = p.state + ((int64_t)unit * np * kUnitRows + sub) * kStateFloats;
-    constexpr int64_t kPiece = (int64_t)kUnitRows * kStateFloats;
-    const int b = bh / p.Hkv, h = bh - b * p.Hkv;
-    float M[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int i = 0; i < np; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) M[r] = fmaxf(M[r], first[i * kPiece + 8 * r * kStateFloats + kHeadDim]);
+    const float* st = p.state + (int64_t)unit * np * kPieceFloats;
+    const int ml = kPieceML + 2 * (wave * kPfQ + n), oo = ((wave * 16 + 4 * db) * 64 + lane) * 4;
+    float M = -INFINITY;
+#pragma unroll 4
+    for (int i = 0; i < np; ++i) M = fmaxf(M, st[(int64_t)i * kPieceFloats + ml]);
     pf4 O[4] = {};
-    float L[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int i = 0; i < np; ++i)
+    float L = 0.f;
+#pragma unroll 4
+    for (int i = 0; i < np; ++i) {
+        const float* s = st + (int64_t)i * kPieceFloats;
+        const float2 x = *(const float2*)(s + ml);
+        const float e = x.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x.x - M);
+        L += x.y * e;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float* st = first + i * kPiece + 8 * r * kStateFloats;
-            const float2 x = *(const float2*)(st + kHeadDim);
-            const pf4 o = *(const pf4*)(st + d);
-            const float e = x.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x.x - M[r]);
-            L[r] += x.y * e;
-            O[r] += o * e;
-        }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = unit_row(p, rb, sub + 8 * r);
-        if (row >= p.Sq * p.nrep) continue;
-        uint16_t* op = p.out + (int64_t)b * p.o_sb + (int64_t)(h * p.nrep + row % p.nrep) * p.o_sh +
-                       (int64_t)(row / p.nrep) * p.o_st;
-        store_out4(p, op + d, O[r], L[r] > 0.f ? 1.0f / L[r] : 0.f);
+        for (int j = 0; j < 4; ++j) O[j] += *(const pf4*)(s + oo + j * 256) * e;
     }
+    if (row >= p.Sq * p.nrep) return;
+    const int b = bh / p.Hkv, h = bh - b * p.Hkv;
+    uint16_t* op = p.out + (int64_t)b * p.o_sb + (int64_t)(h * p.nrep + row % p.nrep) * p.o_sh +
+                   (int64_t)(row / p.nrep) * p.o_st;
+    const float inv = L > 0.f ? 1.0f / L : 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) store_out4(p, op + 32 * db + 8 * j + 4 * hh, O[j], inv);
 }
 
 // ---- the work plan (host)
@@ -284,10 +298,11 @@ size_t chunk_ws_bytes(const HkvPrefillArgs* a) {
     return 2 * (size_t)a->batch * a->num_kv_heads * ccap * kHeadDim * 2;
 }
 
-int launch_attn(PrefillParams& p, const Plan& pl, hipStream_t stream) {
-    static void (*const fns[4])(PrefillParams) = {nullptr, prefill_attn_kernel<1>, prefill_attn_kernel<2>,
-                                                  prefill_attn_kernel<3>};
-    static std::atomic<uint64_t> raised[4];   // four tile buffers exceed the 64 KB default
+int launch_attn(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream) {
+    static void (*const fns[9])(PrefillParams) = {
+        nullptr, prefill_attn_kernel<1>, prefill_attn_kernel<2>, prefill_attn_kernel<3>, prefill_attn_kernel<4>,
+        nullptr, nullptr, nullptr, prefill_attn_kernel<8>};
+    static std::atomic<uint64_t> raised[9];   // four tile buffers exceed the 64 KB default
     p.units = pl.units;
     p.finish = pl.finish;
     const unsigned all = (unsigned)(p.B * p.Hkv * p.units);
@@ -298,6 +313,7 @@ int launch_attn(PrefillParams& p, const Plan& pl, hipStream_t stream) {
             p.pieces[k] = serial && k != kind ? 0 : pl.pieces[k];
             if (p.pieces[k] > 0) kinds |= 1 << k;
         }
+        if (ref) kinds = 1 << (p.int4_max_len % 4 == 0 ? kKindRefVec : kKindRef);
         HKV_RAISE_LDS(fns[kinds], kFlatLdsBytes, raised[kinds]);
         hipLaunchKernelGGL(fns[kinds], dim3(all * (unsigned)(p.pieces[0] + p.pieces[1])), dim3(kFlatThreads),
                            kFlatLdsBytes, stream, p);
@@ -315,8 +331,9 @@ int launch_attn(PrefillParams& p, const Plan& pl, hipStream_t stream) {
 
 using namespace hkv;
 
-extern "C" int hkv_prefill_attn(const HkvPrefillArgs* a, void* stream) {
-    clear_error();
+// The launch behind both entry points; `ref` is null, or holds the INT4 tokens in place of
+// the pool.
+static int prefill_launch(const HkvPrefillArgs* a, const PfRefSource* ref, void* stream) {
     HKV_REQUIRE(a != nullptr, HKV_ERR_ARG, "hkv_prefill_attn: null args");
     HKV_REQUIRE(a->head_dim == kHeadDim, HKV_ERR_UNSUPPORTED, "hkv_prefill_attn: head_dim %d != 128", a->head_dim);
     HKV_REQUIRE(a->batch > 0 && a->num_kv_heads > 0 && a->num_q_heads > 0 && a->num_queries > 0, HKV_ERR_ARG,
@@ -344,7 +361,7 @@ extern "C" int hkv_prefill_attn(const HkvPrefillArgs* a, void* stream) {
                     HKV_ERR_ARG, "hkv_prefill_attn: chunk K/V must be 16-byte aligned, strides multiple of 8");
     }
     HKV_REQUIRE(a->int4_max_len >= 0, HKV_ERR_ARG, "hkv_prefill_attn: int4_max_len < 0");
-    if (a->int4_max_len > 0) {
+    if (a->int4_max_len > 0 && !ref) {
         HKV_REQUIRE(a->block_table && ((a->pool && a->pool_blocks > 0) || (a->staging && a->staging_blocks > 0)),
                     HKV_ERR_ARG, "hkv_prefill_attn: INT4 zone without pool/staging records or block table");
         HKV_REQUIRE(a->pool_blocks >= 0 && a->staging_blocks >= 0 && a->staging_blocks <= (1ll << 31),
@@ -399,6 +416,7 @@ extern "C" int hkv_prefill_attn(const HkvPrefillArgs* a, void* stream) {
     p.bt_stride = a->bt_stride;
     p.int4_lens = a->int4_lens;
     p.int4_max_len = a->int4_max_len;
+    p.ref = ref ? *ref : PfRefSource{};
     p.out = a->out;
     p.o_sb = a->out_stride_b;
     p.o_sh = a->out_stride_h;
@@ -447,7 +465,55 @@ extern "C" int hkv_prefill_attn(const HkvPrefillArgs* a, void* stream) {
     const int64_t rows = ws_ok && a->workspace_bytes > chunk_bytes
                              ? (int64_t)((a->workspace_bytes - chunk_bytes) / (kStateFloats * sizeof(float)))
                              : 0;
-    return launch_attn(p, plan_of(a, rows), (hipStream_t)stream);
+    return launch_attn(p, plan_of(a, rows), ref != nullptr, (hipStream_t)stream);
+}
+
+extern "C" int hkv_prefill_attn(const HkvPrefillArgs* a, void* stream) {
+    clear_error();
+    return prefill_launch(a, nullptr, stream);
+}
+
+// The prefill call that a fused forward makes: its INT4 tokens are all its keys.
+static HkvPrefillArgs fused_as_prefill(const HkvFusedArgs* f) {
+    HkvPrefillArgs a = {};
+    a.batch = f->batch;
+    a.num_q_heads = f->num_q_heads;
+    a.num_kv_heads = f->num_kv_heads;
+    a.head_dim = f->head_dim;
+    a.num_queries = f->num_queries;
+    a.sm_scale = f->sm_scale;
+    a.q = f->q;
+    a.q_stride_b = f->q_stride_b;
+    a.q_stride_h = f->q_stride_h;
+    a.q_stride_t = f->q_stride_t;
+    a.int4_max_len = f->num_tokens;
+    a.out = f->out;
+    a.out_stride_b = f->out_stride_b;
+    a.out_stride_h = f->out_stride_h;
+    a.out_stride_t = f->out_stride_t;
+    a.err_flag = f->err_flag;
+    a.q_dtype = f->q_dtype;
+    a.out_dtype = f->out_dtype;
+    a.workspace = f->workspace;
+    a.workspace_bytes = f->workspace_bytes;
+    return a;
+}
+
+extern "C" int hkv_fused_forward(const HkvFusedArgs* f, void* stream) {
+    clear_error();
+    HKV_REQUIRE(f != nullptr, HKV_ERR_ARG, "hkv_fused_forward: null args");
+    HKV_REQUIRE(f->num_tokens >= 0, HKV_ERR_ARG, "hkv_fused_forward: num_tokens < 0");
+    const int rc = check_fused_source(f, "hkv_fused_forward");
+    if (rc != HKV_OK) return rc;
+    const HkvPrefillArgs a = fused_as_prefill(f);
+    const PfRefSource ref = {f->k_codes, f->v_codes, f->k_scales, f->v_scales, f->k_zps, f->v_zps};
+    return prefill_launch(&a, f->num_tokens > 0 ? &ref : nullptr, stream);
+}
+
+extern "C" size_t hkv_fused_forward_workspace_bytes(const HkvFusedArgs* f) {
+    if (!f || f->num_tokens < 0) return 0;
+    const HkvPrefillArgs a = fused_as_prefill(f);
+    return hkv_prefill_split_bytes(&a);
 }
 
 extern "C" size_t hkv_prefill_split_bytes(const HkvPrefillArgs* a) {

@@ -45,7 +45,19 @@ constexpr int kPfT = 64;             // tokens per tile
 constexpr float kPfLog2e = 1.4426950408889634f;
 constexpr int kUnitRows = 256;       // rows per unit: 8 waves of kPfQ
 constexpr int kStateFloats = 132;    // a row's state: O[128], m, l, pad
-enum : int { kKindF16 = 0, kKindInt4 = 1 };
+// A piece's states (kFinishPieces) in the room of 256 rows: O as [wave][16][lane] 16-byte
+// pieces (piece 4 db + j of lane (n, hh): dims 32 db + 8 j + 4 hh .. +3 of row 32 wave + n),
+// so that both kernels move whole kilobytes, then (m, l) per row.
+constexpr int kPieceFloats = kUnitRows * kStateFloats, kPieceML = kUnitRows * kHeadDim;
+// kKindRef, kKindRefVec: INT4 tiles from unpacked codes, rows of any or of 4 k tokens
+enum : int { kKindF16 = 0, kKindInt4 = 1, kKindRef = 2, kKindRefVec = 3 };
+// INT4 keys and values in the unpacked reference layout: one byte per code, [batch][kv
+// head][int4_max_len][128], with a float scale and a byte zero point per row.
+struct PfRefSource {
+    const uint8_t *kc, *vc;
+    const float *ks, *vs;
+    const uint8_t *kz, *vz;
+};
 
 // Where the fp16 tiles of one source lie (a zone, or the causal chunk in
 // the zone layout): K rows [B*Hkv][cap][128], V tiles [B*Hkv][cap/16][16 x 128].
@@ -79,6 +91,7 @@ struct PrefillParams {
     int bt_stride;
     const int32_t* int4_lens;
     int int4_max_len;
+    PfRefSource ref;             // the INT4 tokens of the fused entry point (no pool then)
     uint16_t* out;
     int64_t o_sb, o_sh, o_st;
     int* err;
@@ -103,10 +116,10 @@ __device__ __forceinline__ int unit_last_row(const PrefillParams& p, int rb) {
     return min((halves - rb) * kHalf, p.Sq * p.nrep) - 1;
 }
 
-// First state row of piece s of kind `kind` of unit `unit` (counted over all pairs).
-__device__ __forceinline__ int64_t piece_row(const PrefillParams& p, int kind, int unit, int s) {
+// The states of piece s of kind `kind` of unit `unit` (counted over all pairs).
+__device__ __forceinline__ float* piece_state(const PrefillParams& p, int kind, int unit, int s) {
     const int per_unit = p.pieces[0] + p.pieces[1];
-    return ((int64_t)unit * per_unit + (kind == kKindInt4 ? s : p.pieces[kKindInt4] + s)) * kUnitRows;
+    return p.state + ((int64_t)unit * per_unit + (kind == kKindInt4 ? s : p.pieces[kKindInt4] + s)) * kPieceFloats;
 }
 
 // Tile counts of one sequence: INT4 tiles, each zone's tiles, and the causal chunk's

@@ -1,5 +1,5 @@
 // The staging policies of the chunked-prefill tile loop: fp16 zone and chunk tiles
-// (F16Stage) and INT4 tiles of the block pool (Int4Stage).  Waves 0-3 of a workgroup (team
+// (F16Stage), INT4 tiles of the block pool (Int4Stage) and of unpacked codes (RefStage).  Waves 0-3 of a workgroup (team
 // 0) stage a tile's K rows, waves 4-7 (team 1) its V^T rows, 16 tokens per wave.
 #pragma once
 
@@ -39,6 +39,9 @@ __device__ __forceinline__ int block_id4(const PrefillParams& p, int nb, int b, 
     const int lb = min(x * 4 + wt, nb - 1);
     return p.bt[(int64_t)b * p.bt_stride + lb];
 }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
 // Buffer resource over this wave's head part of record `id` (an out-of-range id is
 // reported and replaced by a valid record).  The range check is a 32-bit unsigned
 // compare of a wave-uniform value, and the id used is read back from lane 0, so it and
@@ -52,7 +55,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t part_rsrc(const PrefillParams&
     const int64_t rb = (int64_t)p.Hkv * kHeadPartBytes;
     const uint8_t* part = (phys >= 0 ? p.pool + (int64_t)phys * rb : p.staging + (int64_t)(~phys) * rb) +
                           RecordLayout::part(h);
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(part), 0, kHeadPartBytes, 0x00020000);
+    return buf_rsrc(part, kHeadPartBytes);
 }
 __device__ __forceinline__ u4 bld16(__amdgpu_buffer_rsrc_t r, int off) {
     return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
@@ -223,7 +226,7 @@ struct F16Stage {
         // 16-token tile (4 KB), lane i bytes 64 i: halves [n][i] = V[4g + i][c + 16n]
         const int bytes = kTeam == 0 ? nv * (kHeadDim * 2)
                                      : (nv + kBlockTokens - 1) / kBlockTokens * (kBlockTokens * kHeadDim * 2);
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(base, bytes);
         const int off = w.wt * (kBlockTokens * kHeadDim * 2) + w.lane * 64;
 #pragma unroll
         for (int j = 0; j < 4; ++j) dst[j] = bld16(r, off + 16 * j);
@@ -281,6 +284,120 @@ struct F16Stage {
                     if (tb * 32 + 8 * (r >> 2) + 4 * w.hh + (r & 3) > lim) S[tb][r] = -INFINITY;
         }
     }
+};
+
+// The staging policy of unpacked INT4 codes: the same staged values as Int4Stage, from one
+// byte per code.  Reading the codes directly, twice the packed bytes, costs less than
+// clearing a pool, repacking the codes into it and reading that (512 queries of 32/32 heads
+// over 4096 keys: 90 -> 64 us a call).  A tile takes ~7% longer than a packed one: twice the
+// code words to load and unpack.  kVec: rows of a multiple of 4 tokens, whose scales and zero
+// points load as vectors, which leaves registers for a second tile in flight.
+template <int kTeam, bool kVec>
+struct RefStage {
+    static constexpr int kRing = kVec ? 2 : 1;
+    const PrefillParams& p;
+    const FlatWave& w;
+    const int x0, len;     // the unit's tiles from x0, tokens up to len
+    struct Slot {
+        u4 a, b;           // team 0: this lane's 32 K codes; team 1: 4 tokens x (4 + 4) V codes
+        f4 sc;             // scales (team 0: one)
+        uint32_t zp;       // zero points, one per byte
+    } ring[kRing];
+
+    __device__ RefStage(const PrefillParams& p_, const TileMap& tm, const FlatWave& w_, int x0_, int x1_)
+        : p(p_), w(w_), x0(x0_), len(min(tm.len4, x1_ * kPfT)) {}
+    __device__ int tvalid(int x) const { return min(kPfT, max(0, len - (x0 + x) * kPfT)); }
+    // Requests tile x.  The resources end with its valid rows: what lies past them reads as
+    // zero (scale 0: staged as zeros).
+    __device__ void load(int x, Slot& s) const {
+        const int nv = tvalid(x);
+        const int64_t row = ((int64_t)w.b * p.Hkv + w.h) * p.int4_max_len + (int64_t)(x0 + x) * kPfT;
+        const uint8_t *codes = kTeam == 0 ? p.ref.kc : p.ref.vc, *zps = kTeam == 0 ? p.ref.kz : p.ref.vz;
+        const float* scales = kTeam == 0 ? p.ref.ks : p.ref.vs;
+        const __amdgpu_buffer_rsrc_t rc = buf_rsrc(codes + row * kHeadDim, nv * kHeadDim);
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(scales + row, nv * 4), rz = buf_rsrc(zps + row, nv);
+        if constexpr (kTeam == 0) {
+            // token 16 wt + lane / 4, dims 32 (lane % 4) .. +32
+            const int tok = w.wt * 16 + (w.lane >> 2), off = tok * kHeadDim + (w.lane & 3) * 32;
+            s.a = bld16(rc, off);
+            s.b = bld16(rc, off + 16);
+            s.sc[0] = __uint_as_float(bld4(rs, tok * 4));
+            s.zp = __builtin_amdgcn_raw_buffer_load_b8(rz, tok, 0, 0);
+        } else {
+            // tokens 16 wt + 4g .. +3, dims 4c .. +3 and 64 + 4c .. +3 (g = lane / 16, c = lane % 16)
+            const int t0 = w.wt * 16 + (w.lane >> 4) * 4, off = t0 * kHeadDim + (w.lane & 15) * 4;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                s.a[t] = bld4(rc, off + t * kHeadDim);
+                s.b[t] = bld4(rc, off + t * kHeadDim + 64);
+            }
+            if constexpr (kVec) {
+                s.sc = __builtin_bit_cast(f4, bld16(rs, t0 * 4));
+                s.zp = bld4(rz, t0);
+            } else {
+                s.zp = 0u;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    s.sc[t] = __uint_as_float(bld4(rs, (t0 + t) * 4));
+                    s.zp |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(rz, t0 + t, 0, 0) << (8 * t);
+                }
+            }
+        }
+    }
+    // (code - zero point) x scale as Int4Stage stages it: the scale rounded to fp16, then the
+    // product.  Only the low four bits of a code count, as in the packed pool.
+    __device__ void stage(int slot, uint8_t* buf, uint8_t* bias, int x) const {
+        const Slot& s = ring[slot];
+        if constexpr (kTeam == 0) {
+            const int tok = w.wt * 16 + (w.lane >> 2), pt = w.lane & 3;
+            const _Float16 f = (_Float16)s.sc[0];
+            const fh2 f2 = {f, f}, z = zp1024(s.zp, s.zp);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                u4 o;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t m = (j < 2 ? s.a : s.b)[2 * (j & 1) + e] & 0x0F0F0F0Fu;
+                    const fh2 lo = __builtin_bit_cast(fh2, __builtin_amdgcn_perm(0x64646464u, m, 0x04010400u)) - z;
+                    const fh2 hi = __builtin_bit_cast(fh2, __builtin_amdgcn_perm(0x64646464u, m, 0x04030402u)) - z;
+                    o[2 * e] = __builtin_bit_cast(uint32_t, lo * f2);
+                    o[2 * e + 1] = __builtin_bit_cast(uint32_t, hi * f2);
+                }
+                *(u4*)(buf + k_addr(tok, pt * 4 + j)) = o;
+            }
+            if (pt == 0) ((float*)bias)[tok] = tok < tvalid(x) ? 0.0f : -INFINITY;
+        } else {
+            // lane c's four dims of a word are written starting at the (c / 4)-th: 16 lanes then
+            // write 16 rows on banks of their own (all starting at the first: 4 rows per bank,
+            // 2.25 against 2.0 us per tile)
+            const int unit = w.wt * 4 + (w.lane >> 4), c = w.lane & 15, r = c >> 2;
+            const fh2 z01 = zp1024(s.zp & 0xffu, (s.zp >> 8) & 0xffu), z23 = zp1024((s.zp >> 16) & 0xffu, s.zp >> 24);
+            const fh2 f01 = {(_Float16)s.sc[0], (_Float16)s.sc[1]}, f23 = {(_Float16)s.sc[2], (_Float16)s.sc[3]};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                u4 v = e < 4 ? s.a : s.b;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) v[t] = __builtin_amdgcn_alignbyte(v[t], v[t], r);
+                const uint32_t sel = 0x0C000C00u | (uint32_t)(e & 3) | ((uint32_t)(4 + (e & 3)) << 16);
+                const uint32_t m01 = and_or(__builtin_amdgcn_perm(v[1], v[0], sel), 0x000F000Fu, 0x64006400u);
+                const uint32_t m23 = and_or(__builtin_amdgcn_perm(v[3], v[2], sel), 0x000F000Fu, 0x64006400u);
+                *(u2*)(buf + vt_addr((e < 4 ? 0 : 64) + 4 * c + ((e + r) & 3), unit)) =
+                    u2{__builtin_bit_cast(uint32_t, (__builtin_bit_cast(fh2, m01) - z01) * f01),
+                       __builtin_bit_cast(uint32_t, (__builtin_bit_cast(fh2, m23) - z23) * f23)};
+            }
+        }
+    }
+    __device__ void refill(const TileMap&, int slot, int x) { load(x + kRing, ring[slot]); }
+    __device__ void start(const TileMap&, uint8_t* lds) {
+#pragma unroll
+        for (int x = 0; x < kRing; ++x) load(x, ring[x]);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            stage(x % kRing, flat_buf(lds, x), flat_bias(lds, x), x);
+            load(x + kRing, ring[x % kRing]);
+        }
+    }
+    __device__ void mask(int, pf16v (&)[2]) const {}
 };
 
 }  // namespace hkv

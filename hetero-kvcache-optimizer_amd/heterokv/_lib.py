@@ -168,6 +168,8 @@ SYMBOLS = [
     ("hkv_prefill_split_bytes", ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
     ("hkv_prefill_attn", ctypes.c_int, [ctypes.POINTER(PrefillArgs), vp]),
     ("hkv_fused_decode", ctypes.c_int, [ctypes.POINTER(FusedArgs), vp]),
+    ("hkv_fused_forward", ctypes.c_int, [ctypes.POINTER(FusedArgs), vp]),
+    ("hkv_fused_forward_workspace_bytes", ctypes.c_size_t, [ctypes.POINTER(FusedArgs)]),
     ("hkv_pf_create", ctypes.c_int, [i32, ctypes.c_size_t, i32, ctypes.POINTER(vp)]),
     ("hkv_pf_destroy", ctypes.c_int, [vp]),
     ("hkv_pf_host_ptr", vp, [vp, ctypes.c_size_t]),

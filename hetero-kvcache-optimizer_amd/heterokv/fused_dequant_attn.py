@@ -10,9 +10,8 @@ sm_scale defaulting to 1/sqrt(head_dim).  Unlike the reference's Triton kernel
 exactly that formula, and it also accepts GQA (q heads a multiple of kv heads).
 
 The reference passes unpacked codes (one uint8 per value) with per-token
-scales/zps [B, H, S].  Decode attends them as they are (hkv_fused_decode, the split-K
-decode kernel); forward repacks them into INT4 block records on the device
-(hkv_repack_codes) for the MFMA prefill kernel (hkv_prefill_attn).  q may be fp16 or bf16 (bf16 is narrowed to
+scales/zps [B, H, S], which the kernels attend as they are: the split-K decode kernel
+(hkv_fused_decode) and the MFMA prefill kernel (hkv_fused_forward).  q may be fp16 or bf16 (bf16 is narrowed to
 fp16 operands exactly within the fp16 range).  Device errors (an out-of-range bf16
 value, a decode placement failure) go to a per-device error word that is read without
 blocking at the next call -- a later call raises HeteroKVError -- or at once by
@@ -24,7 +23,7 @@ from typing import Optional
 import torch
 
 from . import _lib, ops
-from ._lib import BLOCK_TOKENS, HeteroKVError
+from ._lib import HeteroKVError
 
 
 _ERR = {}   # device -> ErrorWord shared by the calls on that device
@@ -93,19 +92,6 @@ def fused_dequant_attn_decode(q: torch.Tensor, k_data: torch.Tensor, k_scales: t
     return out.to(q.dtype)
 
 
-def _repack_reference(q, k_data, k_scales, k_zps, v_data, v_scales, v_zps, err):
-    B = q.shape[0]
-    kd, vd = _as_4d(k_data), _as_4d(v_data)
-    Hkv, S = kd.shape[1], kd.shape[2]
-    nblk = (S + BLOCK_TOKENS - 1) // BLOCK_TOKENS
-    pool = ops.Int4Pool(B * nblk, Hkv, q.device)
-    bt = torch.arange(B * nblk, dtype=torch.int32, device=q.device).reshape(B, nblk)
-    start = torch.zeros(B, dtype=torch.int32, device=q.device)
-    ops.repack_codes(pool, kd, vd, k_scales.reshape(B, Hkv, S), v_scales.reshape(B, Hkv, S),
-                     k_zps.reshape(B, Hkv, S), v_zps.reshape(B, Hkv, S), start, bt, err=err)
-    return pool, bt, S
-
-
 def fused_dequant_attn_forward(q: torch.Tensor, k_data: torch.Tensor, k_scales: torch.Tensor,
                                k_zps: torch.Tensor, v_data: torch.Tensor, v_scales: torch.Tensor,
                                v_zps: torch.Tensor, sm_scale: Optional[float] = None) -> torch.Tensor:
@@ -117,9 +103,8 @@ def fused_dequant_attn_forward(q: torch.Tensor, k_data: torch.Tensor, k_scales: 
         sm_scale = 1.0 / math.sqrt(q.shape[-1])
     err = _errword(q.device)
     err.poll()
-    pool, bt, S = _repack_reference(q, k_data, k_scales, k_zps, v_data, v_scales, v_zps, err)
+    kd, vd = _as_4d(k_data), _as_4d(v_data)
     qq = _as_kernel_q(q, err)
-    out = ops.prefill_attention(qq, pool=pool, block_table=bt, int4_max_len=S, sm_scale=sm_scale, err=err,
-                                out_dtype=qq.dtype)
+    out = ops.fused_forward(qq, kd, vd, k_scales, v_scales, k_zps, v_zps, sm_scale, err, qq.dtype)
     err.post()
     return out.to(q.dtype)

@@ -600,6 +600,18 @@ def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale
     return out
 
 
+def fused_forward(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
+    """hkv_fused_forward: attention of q [B, Hq, Sq, 128] over every unpacked token."""
+    a, out, keep = _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype)
+    lib = load()
+    nbytes = lib.hkv_fused_forward_workspace_bytes(ctypes.byref(a))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    if ws is not None:
+        a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
+    check(lib.hkv_fused_forward(ctypes.byref(a), stream_ptr(q.device)), "hkv_fused_forward")
+    return out
+
+
 # ----------------------------------------------------------------------- record gather
 def gather_blocks(src, ids, dst, staging=None, dst_offset=0, err=None):
     """dst record dst_offset + i = record ids[i] of src (ids >= 0) or of staging (~ids[i]).

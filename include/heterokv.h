@@ -445,6 +445,13 @@ typedef struct HkvFusedArgs {
 } HkvFusedArgs;
 
 int hkv_fused_decode(const HkvFusedArgs* args, void* stream);
+/* The same for any number of queries per sequence, every key visible to each
+ * (kernels/fused_dequant_attn.py:371-435), with the numerics of hkv_repack_codes +
+ * hkv_prefill_attn.  flags are ignored.  The workspace may be NULL; with
+ * hkv_fused_forward_workspace_bytes() bytes (0 if the call has no use for one), 16-byte
+ * aligned, a call with too few query rows to fill the GPU splits its keys. */
+int hkv_fused_forward(const HkvFusedArgs* args, void* stream);
+size_t hkv_fused_forward_workspace_bytes(const HkvFusedArgs* args);
 
 /*
  * Host-tier prefetcher (replaces DRAMStorageManager's per-tensor pinned dict,
