@@ -77,17 +77,12 @@ def fused_dequant_attn_decode(q: torch.Tensor, k_data: torch.Tensor, k_scales: t
     kd, vd = _as_4d(k_data), _as_4d(v_data)
     if kd.dim() == 4 and kd.shape[0] != B:
         raise HeteroKVError(-1, "batch mismatch between q and k_data")
-    Hkv, S = kd.shape[1], kd.shape[2]
-    ks = k_scales.reshape(B, Hkv, S)
-    vs = v_scales.reshape(B, Hkv, S)
-    kz = k_zps.reshape(B, Hkv, S)
-    vz = v_zps.reshape(B, Hkv, S)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
     err = _errword(q.device)
     err.poll()
     qq = _as_kernel_q(q, err)
-    out = ops.fused_decode(qq, kd, vd, ks, vs, kz, vz, sm_scale, _WS[q.device], err, qq.dtype)
+    out = ops.fused_decode(qq, kd, vd, k_scales, v_scales, k_zps, v_zps, sm_scale, _WS[q.device], err, qq.dtype)
     err.post()
     return out.to(q.dtype)
 

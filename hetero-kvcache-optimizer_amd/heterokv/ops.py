@@ -18,9 +18,7 @@ _DTYPES = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16, torch
 
 def _require_gpu(*ts):
     for t in ts:
-        if t is None:
-            continue
-        if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+        if t is not None and not (isinstance(t, torch.Tensor) and t.is_cuda):
             raise HeteroKVError(-1, "heterokv kernels need tensors on a ROCm GPU (got %s)" %
                                 (t.device if isinstance(t, torch.Tensor) else type(t)))
 
@@ -35,6 +33,7 @@ def _aligned16(t):
 
 
 _F16_OR_BF16 = (torch.float16, torch.bfloat16)
+_SM_SCALE = 1.0 / math.sqrt(HEAD_DIM)
 
 
 class ErrorWord:
@@ -100,11 +99,11 @@ def quantize_groups(x, group_size=128):
     xc = x.contiguous()
     n = xc.numel()
     ng = (n + group_size - 1) // group_size
-    codes = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    scales = torch.empty(ng, dtype=torch.float32, device=x.device)
-    zps = torch.empty(ng, dtype=torch.uint8, device=x.device)
-    check(load().hkv_quantize_groups(_p(xc), _DTYPES[x.dtype], n, group_size, _p(codes), _p(scales),
-                                     _p(zps), stream_ptr(x.device)), "hkv_quantize_groups")
+    codes = xc.new_empty(x.shape, dtype=torch.uint8)
+    scales = xc.new_empty(ng, dtype=torch.float32)
+    zps = xc.new_empty(ng, dtype=torch.uint8)
+    check(load().hkv_quantize_groups(xc.data_ptr(), _DTYPES[x.dtype], n, group_size, codes.data_ptr(),
+                                     scales.data_ptr(), zps.data_ptr(), stream_ptr(x.device)), "hkv_quantize_groups")
     return codes, scales, zps
 
 
@@ -114,7 +113,9 @@ def dequantize_groups(codes, scales, zps, group_size=128, dtype=torch.float16):
     if dtype not in _DTYPES:
         raise HeteroKVError(-1, "dequantize_groups: unsupported dtype %s" % dtype)
     c = codes.contiguous()
-    s = scales.contiguous().to(torch.float32)
+    s = scales.contiguous()
+    if s.dtype != torch.float32:
+        s = s.to(torch.float32)
     z = zps.contiguous()
     if z.dtype != torch.uint8:
         z = z.to(torch.uint8)
@@ -123,9 +124,9 @@ def dequantize_groups(codes, scales, zps, group_size=128, dtype=torch.float16):
     if s.numel() < ng or z.numel() < ng:
         raise HeteroKVError(-3, "dequantize_groups: %d groups need %d scales/zps, got %d/%d" %
                             (ng, ng, s.numel(), z.numel()))
-    out = torch.empty(codes.shape, dtype=dtype, device=codes.device)
-    check(load().hkv_dequantize_groups(_p(c), _p(s), _p(z), n, group_size, _p(out), _DTYPES[dtype],
-                                       stream_ptr(codes.device)), "hkv_dequantize_groups")
+    out = c.new_empty(codes.shape, dtype=dtype)
+    check(load().hkv_dequantize_groups(c.data_ptr(), s.data_ptr(), z.data_ptr(), n, group_size, out.data_ptr(),
+                                       _DTYPES[dtype], stream_ptr(codes.device)), "hkv_dequantize_groups")
     return out
 
 
@@ -475,8 +476,12 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
         out_dtype = q3.dtype if out is None else out.dtype
     if out_dtype not in _F16_OR_BF16:
         raise HeteroKVError(-1, "decode_attention: out dtype must be fp16 or bf16")
-    if q3.stride(-1) != 1 or q3.data_ptr() % 16 or q3.stride(0) % 8 or q3.stride(1) % 8:
+    sb, sh, sd = q3.stride()
+    qp = q3.data_ptr()
+    if sd != 1 or qp % 16 or sb % 8 or sh % 8:
         q3 = q3.contiguous()
+        sb, sh, _ = q3.stride()
+        qp = q3.data_ptr()
     B, Hq, _ = q3.shape
     if len(zones) > _lib.MAX_F16_ZONES:
         raise HeteroKVError(-1, "decode_attention: at most %d fp16 zones" % _lib.MAX_F16_ZONES)
@@ -484,10 +489,10 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
     if Hkv is None:
         raise HeteroKVError(-1, "decode_attention: no key/value zone given")
     if sm_scale is None:
-        sm_scale = 1.0 / math.sqrt(HEAD_DIM)
+        sm_scale = _SM_SCALE
     dev = q3.device
     if out is None:
-        out = torch.empty((B, Hq, HEAD_DIM), dtype=out_dtype, device=dev)
+        out = q3.new_empty((B, Hq, HEAD_DIM), dtype=out_dtype)
     elif out.dtype != out_dtype:
         raise HeteroKVError(-1, "decode_attention: out is %s, out_dtype %s" % (out.dtype, out_dtype))
     a = _lib.DecodeArgs()
@@ -495,7 +500,7 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
     a.err_flag = err.ptr() if err is not None else None
     a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim = B, Hq, Hkv, HEAD_DIM
     a.sm_scale = float(sm_scale)
-    a.q, a.q_stride_b, a.q_stride_h = q3.data_ptr(), q3.stride(0), q3.stride(1)
+    a.q, a.q_stride_b, a.q_stride_h = qp, sb, sh
     a.num_f16_zones = len(zones)
     keep = []
     zl = []
@@ -506,9 +511,10 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
         if lens is not None:
             lt = _i32(lens, dev)
             keep.append(lt)
-        a.f16[i] = _lib.F16Zone(k=z.k.data_ptr(), v=z.v.data_ptr(), capacity=z.capacity, max_len=int(max_len),
-                                lens=lt.data_ptr() if lt is not None else 0)
-        zl.append(int(max_len))
+        max_len = int(max_len)
+        a.f16[i] = _lib.F16Zone(z.k.data_ptr(), z.v.data_ptr(), z.capacity, max_len,
+                                lt.data_ptr() if lt is not None else 0)
+        zl.append(max_len)
     if int4_max_len > 0:
         if (pool is None and staging is None) or block_table is None:
             raise HeteroKVError(-1, "decode_attention: INT4 zone needs a pool and a block table")
@@ -526,12 +532,13 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
             keep.append(il)
             a.int4_lens = il.data_ptr()
     a.int4_max_len = int(int4_max_len)
-    a.out, a.out_stride_b, a.out_stride_h = out.data_ptr(), out.stride(0), out.stride(1)
+    ost = out.stride()
+    a.out, a.out_stride_b, a.out_stride_h = out.data_ptr(), ost[0], ost[1]
     a.splits_hint = int(splits)
     if noalloc:
         a.workspace, a.workspace_bytes = None, 0
     else:
-        nbytes = decode_workspace_bytes(B, Hq, Hkv, int(int4_max_len), zl)
+        nbytes = _decode_workspace_bytes(B, Hq, Hkv, int(int4_max_len), tuple(zl))
         if workspace is None:
             workspace = DecodeWorkspace(dev)
         ws = workspace.get(nbytes)
@@ -559,7 +566,11 @@ def decode_attention(q, zones=(), pool=None, block_table=None, int4_lens=None, i
 # ----------------------------------------------------------------------- fused (unpacked INT4)
 def _row_tensor(t, shape, dtype):
     """t as a contiguous `dtype` tensor of `shape` with a 16-byte aligned base."""
-    t = t.reshape(shape).to(dtype).contiguous()
+    if t.shape != shape:
+        t = t.reshape(shape)
+    if t.dtype != dtype:
+        t = t.to(dtype)
+    t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
@@ -575,12 +586,15 @@ def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale,
     if q.stride(-1) != 1 or q.data_ptr() % 16 or any(st % 8 for st in q.stride()[:3]):
         q = q.contiguous()
     kc, vc = k_codes.contiguous(), v_codes.contiguous()
-    kc, vc = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (kc, vc))
-    ks, vs = (_row_tensor(t, (B, H, T), torch.float32) for t in (k_scales, v_scales))
+    kc = kc if kc.data_ptr() % 16 == 0 else kc.clone()
+    vc = vc if vc.data_ptr() % 16 == 0 else vc.clone()
+    rows = torch.Size((B, H, T))
+    ks, vs = _row_tensor(k_scales, rows, torch.float32), _row_tensor(v_scales, rows, torch.float32)
     # zero points as bytes; other types go through float32, the reference's type for them
-    kz, vz = (_row_tensor(t if t.dtype == k_zps.dtype == torch.uint8 else t.to(torch.float32), (B, H, T), torch.uint8)
-              for t in (k_zps, v_zps))
-    out = torch.empty(q.shape, dtype=out_dtype, device=q.device)
+    if k_zps.dtype != torch.uint8 or v_zps.dtype != torch.uint8:
+        k_zps, v_zps = k_zps.to(torch.float32), v_zps.to(torch.float32)
+    kz, vz = _row_tensor(k_zps, rows, torch.uint8), _row_tensor(v_zps, rows, torch.uint8)
+    out = q.new_empty(q.shape, dtype=out_dtype)
     a = _lib.FusedArgs(batch=B, num_q_heads=q.shape[1], num_kv_heads=H, head_dim=HEAD_DIM, num_queries=q.shape[2],
                        num_tokens=T, sm_scale=float(sm_scale), q_dtype=_DTYPES[q.dtype], out_dtype=_DTYPES[out_dtype],
                        q=q.data_ptr(), q_stride_b=q.stride(0), q_stride_h=q.stride(1), q_stride_t=q.stride(2),
@@ -593,7 +607,7 @@ def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale,
 def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, workspace, err, out_dtype):
     """hkv_fused_decode: decode attention (q [B, Hq, 1, 128]) straight from unpacked codes."""
     a, out, keep = _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype)
-    ws = workspace.get(decode_workspace_bytes(a.batch, a.num_q_heads, a.num_kv_heads, a.num_tokens, ()))
+    ws = workspace.get(_decode_workspace_bytes(a.batch, a.num_q_heads, a.num_kv_heads, a.num_tokens, ()))
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     a.flags = _lib.DECODE_AGENT_HANDOFF if workspace.agent_handoff else 0
     check(load().hkv_fused_decode(ctypes.byref(a), stream_ptr(q.device)), "hkv_fused_decode")
