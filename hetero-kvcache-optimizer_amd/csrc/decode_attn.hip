@@ -863,23 +863,21 @@ enum : int { kSrcPool = 0, kSrcRef = 1, kSrcRefVec = 2 };   // unpacked layout; 
 template <bool kDynamic, bool kScores, bool kL2, bool kShared, int kSrc = kSrcPool>
 __global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
     touch_kernel_args(p);   // the range plan below reads the arguments in a dependent chain
-    int b, h, split, nsplit, first = 0;
+    int bh, split, nsplit, first = 0;
     if constexpr (kShared) {
         const RangePlan r = share_ranges(p, (int)blockIdx.x / p.Hkv);
         if (r.nsplit == 0) return;   // a range left over
-        b = r.b;
-        h = (int)blockIdx.x % p.Hkv;
+        bh = r.b * p.Hkv + (int)blockIdx.x % p.Hkv;
         split = r.split;
         nsplit = r.nsplit;
         first = r.first;
     } else {
-        const int BH = p.B * p.Hkv, pair = blockIdx.x % BH;
-        b = pair / p.Hkv;
-        h = pair % p.Hkv;
+        const int BH = p.B * p.Hkv;
+        bh = blockIdx.x % BH;
         split = blockIdx.x / BH;
         nsplit = p.max_splits;
     }
-    const int bh = b * p.Hkv + h;
+    const int b = bh / p.Hkv, h = bh % p.Hkv;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: buffer resources stay scalar
     const int c = lane & 15, g = lane >> 4;

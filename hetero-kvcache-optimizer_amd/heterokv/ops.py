@@ -134,14 +134,17 @@ def dequantize_groups(codes, scales, zps, group_size=128, dtype=torch.float16):
 class Int4Pool:
     """Device array of INT4 block records: uint8 [num_blocks, record_bytes]."""
 
-    def __init__(self, num_blocks, num_kv_heads, device, head_dim=HEAD_DIM):
+    def __init__(self, num_blocks, num_kv_heads, device, head_dim=HEAD_DIM, fill=True, err=None):
+        """fill=False: records with unspecified contents, for a caller that writes every token it
+        attends; err: the device int32 that reports errors (default: one of the pool's own)."""
         if head_dim != HEAD_DIM:
             raise HeteroKVError(-4, "Int4Pool: head_dim must be 128")
         self.num_kv_heads = num_kv_heads
         self.record_bytes = record_bytes(num_kv_heads)
         self.num_blocks = num_blocks
-        self.data = torch.zeros((max(num_blocks, 1), self.record_bytes), dtype=torch.uint8, device=device)
-        self.err = torch.zeros(1, dtype=torch.int32, device=device)
+        alloc = torch.zeros if fill else torch.empty
+        self.data = alloc((max(num_blocks, 1), self.record_bytes), dtype=torch.uint8, device=device)
+        self.err = torch.zeros(1, dtype=torch.int32, device=device) if err is None else err
 
     @property
     def device(self):
@@ -614,8 +617,36 @@ def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale
     return out
 
 
+# Query rows per kv head, and query-token products of the call, from which fused_forward repacks
+# the codes: a tile of unpacked codes takes the prefill kernel longer, once per 256 rows, and
+# repacking costs one pass over the codes and some launches.  What each route takes above the
+# prefill kernel on repacked records alone (both include the error word's copy), direct and
+# repacked, in us: 32/8 heads, 1024 queries over 1024 tokens 0.6 and 7.4, over 16001 (5.2e8
+# products) 12.1 and 8.2; 2048 queries over 6260 (4.1e8) 3.4 and 8.7, over 16001 (1.0e9) 33 and
+# 8.0; 28/4 heads, 1024 queries over 6260 (1.8e8) 9.5 and 12.9; four sequences of 32/8 heads,
+# 1765 queries over 1024 (2.3e8) 11.0 and 8.3, over 6260 (1.4e9) 38 and 3.8.
+_REPACK_ROWS = 3072
+_REPACK_WORK = 1 << 28
+
+
+def _repacks(batch, q_heads, kv_heads, queries, tokens):
+    rows = queries * (q_heads // kv_heads) if kv_heads else 0
+    return rows >= _REPACK_ROWS and batch * q_heads * queries * tokens >= _REPACK_WORK
+
+
 def fused_forward(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
-    """hkv_fused_forward: attention of q [B, Hq, Sq, 128] over every unpacked token."""
+    """Attention of q [B, Hq, Sq, 128] over every unpacked token: hkv_fused_forward, or with
+    many query rows and tokens hkv_repack_codes and hkv_prefill_attn."""
+    if q.dim() == 4 and k_codes.dim() == 4 and _repacks(q.shape[0], q.shape[1], k_codes.shape[1], q.shape[2],
+                                                        k_codes.shape[2]):
+        B, H, T, _ = k_codes.shape
+        nblk = (T + BLOCK_TOKENS - 1) // BLOCK_TOKENS
+        pool = Int4Pool(B * nblk, H, q.device, fill=False, err=err.dev)
+        bt = torch.arange(B * nblk, dtype=torch.int32, device=q.device).reshape(B, nblk)
+        start = torch.zeros(B, dtype=torch.int32, device=q.device)
+        repack_codes(pool, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, start, bt, err=err)
+        return prefill_attention(q, pool=pool, block_table=bt, int4_max_len=T, sm_scale=sm_scale, err=err,
+                                 out_dtype=out_dtype)
     a, out, keep = _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype)
     lib = load()
     nbytes = lib.hkv_fused_forward_workspace_bytes(ctypes.byref(a))

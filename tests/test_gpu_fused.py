@@ -90,3 +90,15 @@ def test_fused_forward_split_keys(hkv, S, Sq):
     print("case: fused forward split %d heads S=%d Sq=%d" % (hkv, S, Sq), flush=True)
     x = _inputs(9, 1, hkv, hkv, S, Sq, torch.float16)
     _check(fused_dequant_attn_forward(x[0].to(DEV), *[_dev(t) for t in x[1:]]), _reference(*x), torch.float16)
+
+
+@pytest.mark.parametrize("hq,hkv,S,Sq", [(12, 1, 70, 255), (12, 1, 70, 256), (12, 1, 33, 257)])
+def test_fused_forward_row_rule(hq, hkv, S, Sq, monkeypatch):
+    """Query rows per kv head on both sides of the line at which the codes are repacked (into a
+    pool whose last block is written only in part), without the line on the call's work."""
+    from heterokv import fused_dequant_attn_forward, ops
+    monkeypatch.setattr(ops, "_REPACK_WORK", 0)
+    assert ops._repacks(2, hq, hkv, Sq, S) == (Sq >= 256)
+    print("case: fused forward rows %d" % (hq // hkv * Sq), flush=True)
+    x = _inputs(11, 2, hq, hkv, S, Sq, torch.float16)
+    _check(fused_dequant_attn_forward(x[0].to(DEV), *[_dev(t) for t in x[1:]]), _reference(*x), torch.float16)
