@@ -577,15 +577,21 @@ def _row_tensor(t, shape, dtype):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
-    """(FusedArgs, out, tensors to keep) of one call: q [B, Hq, Sq, 128], codes uint8
-    [B, Hkv, S, 128], scales / zps [B, Hkv, S]."""
+def _check_fused(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps):
+    """What every route of a fused call needs, checked before one is taken: q [B, Hq, Sq, 128],
+    codes [B, Hkv, S, 128] of the same batch (the kernels index the codes, or the block table
+    made from them, by q's sequences)."""
     _require_gpu(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps)
-    B, H, T, D = k_codes.shape
-    if D != HEAD_DIM or v_codes.shape != k_codes.shape:
+    if k_codes.dim() != 4 or k_codes.shape[-1] != HEAD_DIM or v_codes.shape != k_codes.shape:
         raise HeteroKVError(-1, "fused attention: codes must be [B, H, T, 128]")
-    if q.dtype not in _F16_OR_BF16 or q.dim() != 4 or q.shape[-1] != HEAD_DIM or q.shape[0] != B:
+    if q.dtype not in _F16_OR_BF16 or q.dim() != 4 or q.shape[-1] != HEAD_DIM or q.shape[0] != k_codes.shape[0]:
         raise HeteroKVError(-1, "fused attention: q must be fp16 or bf16 [B, Hq, Sq, 128]")
+
+
+def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
+    """(FusedArgs, out, tensors to keep) of one call that _check_fused let pass: q [B, Hq, Sq, 128],
+    codes uint8 [B, Hkv, S, 128], scales / zps [B, Hkv, S]."""
+    B, H, T, _ = k_codes.shape
     if q.stride(-1) != 1 or q.data_ptr() % 16 or any(st % 8 for st in q.stride()[:3]):
         q = q.contiguous()
     kc, vc = k_codes.contiguous(), v_codes.contiguous()
@@ -609,6 +615,7 @@ def _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale,
 
 def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, workspace, err, out_dtype):
     """hkv_fused_decode: decode attention (q [B, Hq, 1, 128]) straight from unpacked codes."""
+    _check_fused(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps)
     a, out, keep = _fused_args(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype)
     ws = workspace.get(_decode_workspace_bytes(a.batch, a.num_q_heads, a.num_kv_heads, a.num_tokens, ()))
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
@@ -637,9 +644,9 @@ def _repacks(batch, q_heads, kv_heads, queries, tokens):
 def fused_forward(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
     """Attention of q [B, Hq, Sq, 128] over every unpacked token: hkv_fused_forward, or with
     many query rows and tokens hkv_repack_codes and hkv_prefill_attn."""
-    if q.dim() == 4 and k_codes.dim() == 4 and _repacks(q.shape[0], q.shape[1], k_codes.shape[1], q.shape[2],
-                                                        k_codes.shape[2]):
-        B, H, T, _ = k_codes.shape
+    _check_fused(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps)
+    B, H, T, _ = k_codes.shape
+    if _repacks(B, q.shape[1], H, q.shape[2], T):
         nblk = (T + BLOCK_TOKENS - 1) // BLOCK_TOKENS
         pool = Int4Pool(B * nblk, H, q.device, fill=False, err=err.dev)
         bt = torch.arange(B * nblk, dtype=torch.int32, device=q.device).reshape(B, nblk)

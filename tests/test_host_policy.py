@@ -117,3 +117,23 @@ def test_window_selection_follows_score_changes():
     assert m._top_chunks(0, keys, 2) == ("l0_e4", "l0_e5")
     m._chunk_attention_scores["l0_e0"] = 99.0
     assert m._top_chunks(0, keys, 2) == ("l0_e0", "l0_e5")
+
+
+@pytest.mark.parametrize("rows", [1, 1 << 30])
+def test_fused_forward_refuses_another_batch_on_both_routes(monkeypatch, rows):
+    """Queries of more sequences than the codes are refused before either route (the block
+    table made for the codes has no row for them): no pool is made, no kernel is reached."""
+    from heterokv import HeteroKVError, ops
+    reached = []
+    monkeypatch.setattr(ops, "_require_gpu", lambda *ts: None)
+    monkeypatch.setattr(ops, "_REPACK_ROWS", rows)
+    monkeypatch.setattr(ops, "_REPACK_WORK", 0)
+    for name in ("Int4Pool", "repack_codes", "prefill_attention", "load"):
+        monkeypatch.setattr(ops, name, lambda *a, _n=name, **k: reached.append(_n))
+    q = torch.zeros((2, 4, 8, 128), dtype=torch.float16)
+    codes, rows_ = torch.zeros((1, 2, 32, 128), dtype=torch.uint8), torch.zeros((1, 2, 32))
+    assert ops._repacks(2, 4, 2, 8, 32) == (rows == 1)
+    with pytest.raises(HeteroKVError, match="q must be"):
+        ops.fused_forward(q, codes, codes, rows_, rows_, rows_, rows_, 1.0, SimpleNamespace(dev=None, ptr=lambda: 0),
+                          torch.float16)
+    assert reached == []
