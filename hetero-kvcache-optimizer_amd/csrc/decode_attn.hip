@@ -171,7 +171,6 @@ struct DecodeParams {
     int bt_stride;
     const int32_t* int4_lens;
     int int4_max_len;
-    RefSource ref;
     uint16_t* out;
     int64_t o_sb, o_sh;
     int* err;
@@ -201,6 +200,25 @@ struct DecodeParams {
     int tl_waits;              // 1: also wait for the prologue loads and stamp their arrival
 #endif
 };
+// The unpacked layout's kernels take its source behind the common arguments.  A kernel asks
+// for every line of its arguments before anything else, and the pool's kernels, which never
+// read the source, would ask for seven lines of 64 bytes with it, not six.
+struct RefDecodeParams : DecodeParams {
+    RefSource ref;
+};
+// (a trait on the plain number: a conditional on the kind's enumerator would put the unnamed
+// enumeration into the kernels' mangled names, where host and device number it differently)
+template <int kSrc>
+struct KernelParams {
+    typedef RefDecodeParams type;
+};
+template <>
+struct KernelParams<0> {
+    typedef DecodeParams type;
+};
+#ifndef HKV_DECODE_TIMELINE
+static_assert(sizeof(DecodeParams) <= 6 * 64, "the pool kernels' arguments: six lines");
+#endif
 
 // Partial states cross workgroups (and XCDs) through agent-scope relaxed atomic
 // loads and stores: those are coherent at the device level by themselves, so the
@@ -557,7 +575,7 @@ struct RefBlk {
 // kVec: rows of a multiple of 4 tokens, whose scales and zero points load as vectors.  The
 // resources end with the block's valid rows: what lies past them reads as zero.
 template <bool kVec>
-__device__ __forceinline__ void load_ref(const DecodeParams& p, int64_t bh, int blk, bool valid, int c, int g, RefBlk& d) {
+__device__ __forceinline__ void load_ref(const RefDecodeParams& p, int64_t bh, int blk, bool valid, int c, int g, RefBlk& d) {
     const int64_t row = bh * p.int4_max_len + (int64_t)blk * kBlockTokens;
     const int n = valid ? min(kBlockTokens, p.int4_max_len - blk * kBlockTokens) : 0;
     const __amdgpu_buffer_rsrc_t rk = rsrc(p.ref.kc + row * kHeadDim, n * kHeadDim);
@@ -861,7 +879,7 @@ __device__ __forceinline__ void load_partials(__amdgpu_buffer_rsrc_t prs, const 
 // (in one kernel with it, the 32K decode's launch was 0.25 us longer).  kSrc: where the INT4 tokens are.
 enum : int { kSrcPool = 0, kSrcRef = 1, kSrcRefVec = 2 };   // unpacked layout; vector scales (load_ref)
 template <bool kDynamic, bool kScores, bool kL2, bool kShared, int kSrc = kSrcPool>
-__global__ __launch_bounds__(kThreads) void decode_attn_kernel(DecodeParams p) {
+__global__ __launch_bounds__(kThreads) void decode_attn_kernel(typename KernelParams<kSrc>::type p) {
     touch_kernel_args(p);   // the range plan below reads the arguments in a dependent chain
     int bh, split, nsplit, first = 0;
     if constexpr (kShared) {
@@ -1714,7 +1732,6 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     p.bt_stride = a->bt_stride;
     p.int4_lens = a->int4_lens;
     p.int4_max_len = a->int4_max_len;
-    p.ref = ref ? *ref : RefSource{};
     p.out = a->out;
     p.o_sb = a->out_stride_b;
     p.o_sh = a->out_stride_h;
@@ -1779,23 +1796,35 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     const size_t lds = lds_bytes(nrep);
     const bool det = (a->flags & HKV_DECODE_DETERMINISTIC) != 0;
     const bool sc = a->scores != nullptr;
-    // pool: by schedule, scores, hand-off and range plan; unpacked layout (lengths of its own
-    // do not occur): by hand-off and row alignment
-    const int var = ref ? 16 + (p.xcc_local ? 1 : 0) + (a->int4_max_len % 4 == 0 ? 2 : 0)
-                        : (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0) + (lin > 0 ? 8 : 0);
-#define HKV_DECODE_FN(v) decode_attn_kernel<((v) & 1) != 0, ((v) & 2) != 0, ((v) & 4) != 0, ((v) & 8) != 0>
-#define HKV_DECODE_REF(v) decode_attn_kernel<true, false, ((v) & 1) != 0, false, ((v) & 2) != 0 ? kSrcRefVec : kSrcRef>
-    static void (*const fns[20])(DecodeParams) = {
-        HKV_DECODE_FN(0),  HKV_DECODE_FN(1),  HKV_DECODE_FN(2),  HKV_DECODE_FN(3),  HKV_DECODE_FN(4),
-        HKV_DECODE_FN(5),  HKV_DECODE_FN(6),  HKV_DECODE_FN(7),  HKV_DECODE_FN(8),  HKV_DECODE_FN(9),
-        HKV_DECODE_FN(10), HKV_DECODE_FN(11), HKV_DECODE_FN(12), HKV_DECODE_FN(13), HKV_DECODE_FN(14),
-        HKV_DECODE_FN(15), HKV_DECODE_REF(0), HKV_DECODE_REF(1), HKV_DECODE_REF(2), HKV_DECODE_REF(3)};
-#undef HKV_DECODE_FN
-#undef HKV_DECODE_REF
-    static std::atomic<uint64_t> raised[20];   // the merge area plus the static id window can exceed 64 KB
-    HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
     const dim3 grid((unsigned)(lin > 0 ? (int64_t)a->num_kv_heads * lin : BH * ms)), block(kThreads);
-    hipLaunchKernelGGL(fns[var], grid, block, lds, (hipStream_t)stream, p);
+    // (the merge area plus the static id window can exceed 64 KB of LDS)
+    if (ref) {
+        // unpacked layout (lengths of its own do not occur): by hand-off and row alignment
+#define HKV_DECODE_REF(v) decode_attn_kernel<true, false, ((v) & 1) != 0, false, ((v) & 2) != 0 ? kSrcRefVec : kSrcRef>
+        static void (*const fns[4])(RefDecodeParams) = {HKV_DECODE_REF(0), HKV_DECODE_REF(1), HKV_DECODE_REF(2),
+                                                        HKV_DECODE_REF(3)};
+#undef HKV_DECODE_REF
+        static std::atomic<uint64_t> raised[4];
+        const int var = (p.xcc_local ? 1 : 0) + (a->int4_max_len % 4 == 0 ? 2 : 0);
+        RefDecodeParams rp;
+        static_cast<DecodeParams&>(rp) = p;
+        rp.ref = *ref;
+        HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
+        hipLaunchKernelGGL(fns[var], grid, block, lds, (hipStream_t)stream, rp);
+    } else {
+        // pool: by schedule, scores, hand-off and range plan
+#define HKV_DECODE_FN(v) decode_attn_kernel<((v) & 1) != 0, ((v) & 2) != 0, ((v) & 4) != 0, ((v) & 8) != 0>
+        static void (*const fns[16])(DecodeParams) = {
+            HKV_DECODE_FN(0),  HKV_DECODE_FN(1),  HKV_DECODE_FN(2),  HKV_DECODE_FN(3),
+            HKV_DECODE_FN(4),  HKV_DECODE_FN(5),  HKV_DECODE_FN(6),  HKV_DECODE_FN(7),
+            HKV_DECODE_FN(8),  HKV_DECODE_FN(9),  HKV_DECODE_FN(10), HKV_DECODE_FN(11),
+            HKV_DECODE_FN(12), HKV_DECODE_FN(13), HKV_DECODE_FN(14), HKV_DECODE_FN(15)};
+#undef HKV_DECODE_FN
+        static std::atomic<uint64_t> raised[16];
+        const int var = (det ? 0 : 1) + (sc ? 2 : 0) + (p.xcc_local ? 4 : 0) + (lin > 0 ? 8 : 0);
+        HKV_RAISE_LDS(fns[var], 96 * 1024, raised[var]);
+        hipLaunchKernelGGL(fns[var], grid, block, lds, (hipStream_t)stream, p);
+    }
     HKV_LAUNCH_CHECK("decode_attn_kernel");
     return HKV_OK;
 }
