@@ -298,13 +298,39 @@ size_t chunk_ws_bytes(const HkvPrefillArgs* a) {
     return 2 * (size_t)a->batch * a->num_kv_heads * ccap * kHeadDim * 2;
 }
 
-int launch_attn(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream) {
+// Sequences b0 .. b0 + n - 1 of a launch.  The state rows are used again by every slice: the
+// stream orders a slice's kernels after those of the one before.
+PrefillParams batch_slice(const PrefillParams& p, int b0, int n) {
+    PrefillParams s = p;
+    const int64_t pairs = (int64_t)b0 * p.Hkv, codes = pairs * p.int4_max_len;
+    s.B = n;
+    s.q += b0 * p.q_sb;
+    s.out += b0 * p.o_sb;
+    for (const int32_t*& l : s.zone_lens)
+        if (l) l += b0;
+    for (PfSrc& f : s.src)
+        if (f.k) {
+            f.k += pairs * f.cap * kHeadDim;
+            f.v += pairs * f.cap * kHeadDim;
+        }
+    if (s.bt) s.bt += (int64_t)b0 * p.bt_stride;
+    if (s.int4_lens) s.int4_lens += b0;
+    if (s.ref.kc) {
+        s.ref.kc += codes * kHeadDim;
+        s.ref.vc += codes * kHeadDim;
+        s.ref.ks += codes;
+        s.ref.vs += codes;
+        s.ref.kz += codes;
+        s.ref.vz += codes;
+    }
+    return s;
+}
+
+int launch_slice(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream) {
     static void (*const fns[9])(PrefillParams) = {
         nullptr, prefill_attn_kernel<1>, prefill_attn_kernel<2>, prefill_attn_kernel<3>, prefill_attn_kernel<4>,
         nullptr, nullptr, nullptr, prefill_attn_kernel<8>};
     static std::atomic<uint64_t> raised[9];   // four tile buffers exceed the 64 KB default
-    p.units = pl.units;
-    p.finish = pl.finish;
     const unsigned all = (unsigned)(p.B * p.Hkv * p.units);
     const bool serial = pl.finish == kFinishSerial;
     for (int kind = 0; kind < (serial ? 2 : 1); ++kind) {
@@ -322,6 +348,24 @@ int launch_attn(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream) 
     if (pl.finish == kFinishPieces) {
         hipLaunchKernelGGL(prefill_combine_kernel, dim3(all * kFlatWaves), dim3(256), 0, stream, p);
         HKV_LAUNCH_CHECK("prefill_combine_kernel");
+    }
+    return HKV_OK;
+}
+
+// The pairs and units are all in the grid's x, which takes fewer than 2^32 threads: a call
+// with more goes by slices of its sequences (it has too many units to be split into pieces).
+constexpr int64_t kMaxGridUnits = ((1ll << 32) - 1) / kFlatThreads;
+
+int launch_attn(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream) {
+    p.units = pl.units;
+    p.finish = pl.finish;
+    const int64_t per_seq = (int64_t)p.Hkv * p.units;
+    if (p.B * per_seq <= kMaxGridUnits) return launch_slice(p, pl, ref, stream);
+    const int step = (int)std::max<int64_t>(1, kMaxGridUnits / per_seq);
+    for (int b0 = 0; b0 < p.B; b0 += step) {
+        PrefillParams s = batch_slice(p, b0, std::min(step, p.B - b0));
+        const int rc = launch_slice(s, pl, ref, stream);
+        if (rc != HKV_OK) return rc;
     }
     return HKV_OK;
 }

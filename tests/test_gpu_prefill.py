@@ -295,3 +295,27 @@ def test_paired_half_units(hq, hkv, sq, recent):
     partner, a last one of one row), whose waves stop at different chunk tiles."""
     print("case: paired half-units %d/%d Sq=%d recent %d" % (hq, hkv, sq, recent), flush=True)
     _case(80 + sq, 1, hq, hkv, sq, 0, [0], [recent])
+
+
+def test_more_pairs_than_one_grid_holds():
+    """65535 sequences of 129 heads with one query each: more workgroups of 512 threads than one
+    grid takes (2^32 threads), so the sequences go in two launches.  Sequence b repeats sequence
+    b % 16, whose result is that of a call of 16."""
+    from heterokv import ops
+    B, H = 65535, 129
+    print("case: prefill B=%d %d heads" % (B, H), flush=True)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    pool = ops.Int4Pool(2, H, DEV)
+    kv = torch.randn((1, H, 32, 128), generator=g, device=DEV).half()
+    ops.pack_tokens(pool, kv, kv.flip(2), 0, torch.tensor([[0, 1]], dtype=torch.int32))
+    q = torch.randn((16, H, 1, 128), generator=g, device=DEV).half()
+    lens = torch.arange(1, 17, dtype=torch.int32, device=DEV)
+    bt = (torch.arange(16, dtype=torch.int32, device=DEV) % 2)[:, None]
+    ref = ops.prefill_attention(q, pool=pool, block_table=bt, int4_lens=lens, int4_max_len=16)
+    n = B // 16 + 1
+    out = ops.prefill_attention(q.repeat(n, 1, 1, 1)[:B], pool=pool, block_table=bt.repeat(n, 1)[:B],
+                                int4_lens=lens.repeat(n)[:B], int4_max_len=16)
+    pool.check_errors()
+    full = B // 16 * 16
+    assert torch.equal(out[:full].view(-1, *ref.shape), ref.expand(full // 16, *ref.shape))
+    assert torch.equal(out[full:], ref[:B - full])
