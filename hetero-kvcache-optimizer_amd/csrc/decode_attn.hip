@@ -1484,7 +1484,8 @@ int num_cus() {
 // hand-off: up to kOneRange, two per wave (164 tokens: 5.9 us against 6.8 us), and with the
 // dearer last-arrival merge of fewer than n_rep ranges while s ranges take no more than
 // kOneRangeWide units off one (units (s - 1) / s; pairs for two ranges each, n_rep 4 to 8: 36
-// units 9.9 - 10.9 us in one, 10.5 - 11.2 in two; 49 units 14.4 - 15.1 and 13.4 - 13.9).
+// units 9.9 - 10.9 us in one, 10.5 - 11.2 in two; 49 units 14.4 - 15.1 and 13.4 - 13.9).  That
+// rule weighs s > 1: pairs that take more than half of the CUs go by their length below.
 // Where one round leaves CUs idle that two rounds would use, ranges still long in two (kLongRange bytes) take two (3 sequences of
 // 32/32 heads of 14K to 33K tokens: 2 ranges, 192 workgroups, 106 us; 5 ranges 96 us).
 // Sequences with lengths of their own share the ranges out by length (share_ranges) where an
@@ -1492,6 +1493,11 @@ int num_cus() {
 // of the XCDs the XCD-local hand-off too.  8 sequences of 32/8 heads of 7K to 33K tokens
 // 60.6 -> 51.2 us, 5 of them 42.1 -> 36.1, 3 of 32/32 heads 102 -> 84; of 2K to 9K tokens
 // (even shares of 410 KB) 8 of 32/8 heads 23.2 -> 23.0 and 16 of 28/4 heads 24.6 -> 27.0.
+// With one CU a pair (one range, two, shared out; us): 17 sequences of 32/8 heads of 1K to 9K
+// tokens 53.5, 44.3, 36.1, of 3K to 29K 152, 99, 83; 24 of them 57, 60, 49 and 156, 144, 128; 31
+// 60, 64, 60 and 167, 162, 164; 40 of 28/4 heads 57, 54, 45 and 155, 118, 102.  Two ranges win
+// where few CUs are left over and the lengths differ most (6 sequences of 32/32 heads of 3K to
+// 29K 156, 101, 120; of 14K to 29K 159, 142, 148; of one length 167, 190, 168).
 constexpr int kOneRange = 16, kOneRangeWide = 22;
 constexpr int64_t kLongRange = 512 * 1024;
 
@@ -1513,7 +1519,7 @@ Ranges choose_ranges(int B, int Hkv, int nrep, int int4_max_len, int64_t int4_it
     }
     const int64_t by_units = (units + 1) / 2 > nrep ? (units + 1) / 2 : nrep;
     const int64_t one = cus / BH, two = 2 * cus / BH;
-    if (units <= kOneRange || (one < nrep && units * (one - 1) <= kOneRangeWide * one)) return Ranges{1, 0};
+    if (units <= kOneRange || (one > 1 && one < nrep && units * (one - 1) <= kOneRangeWide * one)) return Ranges{1, 0};
     if (own_lens && B > 1 && B <= 64 && cus / Hkv >= B && bytes >= (one > 0 ? one : 1) * kLongRange) {
         const int64_t lin = cus / Hkv < B * by_units ? cus / Hkv : B * by_units;
         if (lin > B) return Ranges{1, (int)lin};
@@ -1565,6 +1571,26 @@ size_t shared_workspace_bytes(int Hkv, int nrep, int lin) {
     return kTicketAreaEnd + (size_t)Hkv * lin * split_stride_floats(nrep) * sizeof(float);
 }
 
+// The ranges of a checked call with a workspace of ws_bytes: too small a one for the chosen
+// ranges gets fewer.
+Ranges launch_ranges(const HkvDecodeArgs* a, int64_t int4_item_bytes, size_t ws_bytes) {
+    const int nrep = a->num_q_heads / a->num_kv_heads;
+    int32_t zl[HKV_MAX_F16_ZONES] = {0, 0, 0};
+    bool own_lens = a->int4_lens != nullptr;
+    for (int i = 0; i < a->num_f16_zones; ++i) {
+        zl[i] = a->f16[i].max_len;
+        own_lens = own_lens || a->f16[i].lens != nullptr;
+    }
+    Ranges r = choose_ranges(a->batch, a->num_kv_heads, nrep, a->int4_max_len, int4_item_bytes, zl, a->num_f16_zones,
+                             own_lens, a->splits_hint);
+    if (a->splits_hint > 0) return r;
+    const int least = least_splits(a->batch * a->num_kv_heads, a->int4_max_len, int4_item_bytes, zl, a->num_f16_zones);
+    if (r.lin > 0 && shared_workspace_bytes(a->num_kv_heads, nrep, r.lin) > ws_bytes) r = Ranges{least, 0};
+    while (r.per_pair > least && workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, r.per_pair) > ws_bytes)
+        --r.per_pair;
+    return r;
+}
+
 // XCDs that workgroups are dispatched over round-robin: gfx950 has 32 CUs per
 // XCD, so a partition with N CUs spans N / 32 of them.
 int num_xcc() {
@@ -1601,6 +1627,20 @@ extern "C" size_t hkv_decode_workspace_bytes(int32_t batch, int32_t num_q_heads,
         num_f16_zones < 0 || num_f16_zones > HKV_MAX_F16_ZONES || (num_f16_zones > 0 && !f16_max_lens))
         return 0;
     return workspace_bytes(batch, num_q_heads, num_kv_heads, kMaxSplits);
+}
+
+extern "C" int hkv_decode_ranges(const HkvDecodeArgs* a, int32_t* shared) {
+    clear_error();
+    HKV_REQUIRE(a && shared, HKV_ERR_ARG, "hkv_decode_ranges: null pointer");
+    HKV_REQUIRE(a->batch > 0 && a->num_kv_heads > 0 && a->num_q_heads > 0 && a->num_q_heads % a->num_kv_heads == 0 &&
+                    (int64_t)a->batch * a->num_kv_heads < 65536 && a->int4_max_len >= 0 && a->num_f16_zones >= 0 &&
+                    a->num_f16_zones <= HKV_MAX_F16_ZONES,
+                HKV_ERR_ARG, "hkv_decode_ranges: bad sizes");
+    const size_t ws = a->workspace ? a->workspace_bytes
+                                   : workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, kMaxSplits);
+    const Ranges r = launch_ranges(a, kInt4ItemBytes, ws);
+    *shared = r.lin;
+    return r.per_pair;
 }
 
 #ifdef HKV_DECODE_TIMELINE
@@ -1683,19 +1723,8 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
                 "hkv_decode_attn: fp16 zones hold more than %d tokens", kMaxZoneTokens);
     const int64_t BH = (int64_t)a->batch * a->num_kv_heads;
     HKV_REQUIRE(BH < 65536, HKV_ERR_ARG, "hkv_decode_attn: batch x kv heads too large");
-    bool own_lens = a->int4_lens != nullptr;
-    for (int i = 0; i < a->num_f16_zones; ++i) own_lens = own_lens || a->f16[i].lens != nullptr;
-    const Ranges rg = choose_ranges(a->batch, a->num_kv_heads, nrep, a->int4_max_len, ref ? kRefItemBytes : kInt4ItemBytes, zl,
-                                    a->num_f16_zones, own_lens, a->splits_hint);
-    int ms = rg.per_pair, lin = rg.lin;
-    if (a->splits_hint <= 0) {
-        const int least = least_splits((int)BH, a->int4_max_len, ref ? kRefItemBytes : kInt4ItemBytes, zl, a->num_f16_zones);
-        if (lin > 0 && shared_workspace_bytes(a->num_kv_heads, nrep, lin) > ws_bytes) {
-            lin = 0;
-            ms = least;
-        }
-        while (ms > least && workspace_bytes(a->batch, a->num_q_heads, a->num_kv_heads, ms) > ws_bytes) --ms;
-    }
+    const Ranges rg = launch_ranges(a, ref ? kRefItemBytes : kInt4ItemBytes, ws_bytes);
+    const int ms = rg.per_pair, lin = rg.lin;
     HKV_REQUIRE(ms == 1 || BH <= kHandoffPairs, HKV_ERR_CAPACITY,
                 "hkv_decode_attn: %d ranges per pair for %lld (sequence, kv head) pairs; a split launch hands off "
                 "at most %lld pairs", ms, (long long)BH, (long long)kHandoffPairs);

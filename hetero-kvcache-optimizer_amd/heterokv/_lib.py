@@ -163,6 +163,7 @@ SYMBOLS = [
     ("hkv_zone_step", ctypes.c_int, [ctypes.POINTER(ZoneStepArgs), vp]),
     ("hkv_decode_workspace_bytes", ctypes.c_size_t, [i32, i32, i32, i32, i32, vp, i32]),
     ("hkv_decode_attn", ctypes.c_int, [ctypes.POINTER(DecodeArgs), vp]),
+    ("hkv_decode_ranges", ctypes.c_int, [ctypes.POINTER(DecodeArgs), ctypes.POINTER(i32)]),
     ("hkv_decode_attn_noalloc", ctypes.c_int, [ctypes.POINTER(DecodeArgs), vp]),
     ("hkv_prefill_workspace_bytes", ctypes.c_size_t, [i32, i32, i32]),
     ("hkv_prefill_split_bytes", ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),

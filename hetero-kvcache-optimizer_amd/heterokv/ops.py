@@ -400,6 +400,21 @@ def _decode_workspace_bytes(batch, num_q_heads, num_kv_heads, int4_max_len, f16_
     return int(n)
 
 
+def decode_ranges(batch, num_q_heads, num_kv_heads, int4_max_len, zone_max_lens=(), own_lens=False, splits=0):
+    """The library's range plan for a decode call of these sizes (a host query): (ranges per
+    (sequence, kv head) pair, ranges per kv head shared out by the sequences' lengths or 0).
+    own_lens: the call gives per-sequence lengths."""
+    a = _lib.DecodeArgs(batch=batch, num_q_heads=num_q_heads, num_kv_heads=num_kv_heads, head_dim=HEAD_DIM,
+                        int4_max_len=int4_max_len, splits_hint=splits, num_f16_zones=len(zone_max_lens))
+    for i, n in enumerate(zone_max_lens):
+        a.f16[i] = _lib.F16Zone(0, 0, n, n, 0)
+    a.int4_lens = 1 if own_lens else 0   # only whether it is there counts
+    shared = ctypes.c_int32(0)
+    per_pair = load().hkv_decode_ranges(ctypes.byref(a), ctypes.byref(shared))
+    check(min(per_pair, 0), "hkv_decode_ranges")
+    return per_pair, shared.value
+
+
 class DecodeWorkspace:
     """Zero-initialised scratch for hkv_decode_attn; grows on demand (re-zeroed when it
     grows).  Its ticket area has the same offsets for every geometry and the kernels leave

@@ -355,6 +355,13 @@ size_t hkv_decode_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t nu
 
 int hkv_decode_attn(const HkvDecodeArgs* args, void* stream);
 
+/* The range plan of hkv_decode_attn for these sizes (a host query; no kernel runs): returns the
+ * ranges per (sequence, kv head) pair, or 1 with *shared > 0 ranges per kv head that a launch
+ * shares out over its sequences by their lengths.  Reads batch, heads, int4_max_len, the zones'
+ * max_len, splits_hint, and whether int4_lens or a zone's lens are given (never their contents);
+ * workspace NULL stands for one of hkv_decode_workspace_bytes().  Negative: an error code. */
+int hkv_decode_ranges(const HkvDecodeArgs* args, int32_t* shared);
+
 /*
  * hkv_decode_attn without a workspace: no counterpart in the reference.  It is for
  * callers that cannot allocate device memory -- code under HIP graph capture, tight

@@ -137,3 +137,26 @@ def test_fused_forward_refuses_another_batch_on_both_routes(monkeypatch, rows):
         ops.fused_forward(q, codes, codes, rows_, rows_, rows_, rows_, 1.0, SimpleNamespace(dev=None, ptr=lambda: 0),
                           torch.float16)
     assert reached == []
+
+
+@pytest.mark.parametrize("B,hq,hkv,mid,zones,own,want", [
+    # more than half of the CUs' number of pairs: long contexts are shared out by length, or cut
+    # into as many ranges as two rounds hold
+    (17, 32, 8, 9000, (16, 500), True, (1, 32)), (24, 32, 8, 28608, (64, 4096), True, (1, 32)),
+    (31, 32, 8, 9000, (16, 500), True, (1, 32)), (40, 28, 4, 9000, (16, 500), True, (1, 64)),
+    (6, 32, 32, 9000, (16, 500), True, (1, 8)), (17, 32, 8, 28608, (64, 4096), False, (3, 0)),
+    (17, 32, 8, 1000, (16, 100), True, (1, 0)), (24, 32, 8, 28608, (64, 4096), False, (1, 0)),
+    # a pair per CU and more: one range each
+    (32, 32, 8, 28608, (64, 4096), True, (1, 0)), (48, 32, 8, 28608, (64, 4096), True, (1, 0)),
+    # fewer pairs, and few tokens
+    (16, 32, 8, 28608, (64, 4096), True, (1, 32)), (8, 32, 8, 3000, (64, 500), True, (4, 0)),
+    (1, 32, 8, 28608, (64, 4096), False, (32, 0)), (1, 32, 8, 0, (64, 100), False, (1, 0)),
+    (16, 32, 8, 100, (16, 300), True, (1, 0)),
+])
+def test_decode_range_plan(B, hq, hkv, mid, zones, own, want):
+    """The decode launch's range plan on 256 CUs (the library's assumption without a GPU)."""
+    import torch
+    from heterokv import ops
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("a device of another CU count")
+    assert ops.decode_ranges(B, hq, hkv, mid, zones, own_lens=own) == want
