@@ -85,6 +85,9 @@ class Case:
         outs = []
         for b in range(self.B):
             s, m, r = self.sink, self.mids[b], self.recents[b]
+            if s + m + r == 0:   # no key: zeros
+                outs.append(np.zeros((self.Hq, 128)))
+                continue
             parts_k, parts_v = [], []
             if m:
                 kc, ks, kz = oc.compress(self.K[b, :, s:s + m].numpy(), 128)
@@ -384,19 +387,81 @@ def test_range_rule(B, hq, hkv, mid, recent):
     assert ws.error_flag() == 0
 
 
+def _shared_ranges(c):
+    """Ranges per kv head that the library shares out over the case's sequences (0: it does not)."""
+    from heterokv import ops
+    zones = ([c.sink] if c.sink else []) + ([max(c.recents)] if max(c.recents) else [])
+    return ops.decode_ranges(c.B, c.Hq, c.Hkv, c.maxmid, zones, own_lens=c.B > 1)[1]
+
+
 @pytest.mark.parametrize("hq,hkv,mids,recents", [
     (32, 8, [20000, 0, 40, 9000], [100, 0, 300, 17]),     # a sequence without a key but its sink, short and long
-    (28, 4, [70000, 100, 2500], [64, 500, 1]),            # kv heads not a multiple of the XCDs, 64 ranges a pair
+    (28, 4, [70000, 100, 2500], [64, 500, 1]),            # kv heads not a multiple of the XCDs
     (16, 2, [30000] * 5, [33, 200, 1, 90, 64]),           # one length, given per sequence
     (8, 8, [400 + 100 * i for i in range(31)], [20] * 31),   # nearly as many sequences as ranges per head
-    (4, 1, [15000 * (i % 30 == 7) + 5 * i for i in range(64)], [10 + i for i in range(64)]),
 ])
-def test_ranges_shared_by_length(hq, hkv, mids, recents):
-    """Ragged batches, whose ranges are shared out by length, against the oracle, twice on one
-    workspace (the hand-off words come back to rest), then with the device-scope hand-off."""
+def test_ragged_batches(hq, hkv, mids, recents):
+    """Ragged batches whose even share is too short for ranges shared out by length: the same
+    number for every sequence.  Against the oracle, with both hand-offs."""
     from heterokv import ops
-    print("case: shared ranges %d/%d B=%d" % (hq, hkv, len(mids)), flush=True)
+    print("case: ragged %d/%d B=%d" % (hq, hkv, len(mids)), flush=True)
     c = Case(500 + len(mids), len(mids), hq, hkv, 16, mids, recents)
+    assert _shared_ranges(c) == 0
     for ws in (ops.DecodeWorkspace(DEV), ops.DecodeWorkspace(DEV, agent_handoff=True)):
         _check(c, workspace=ws)
         assert ws.error_flag() == 0
+
+
+# kv heads a multiple of the XCDs: the hand-off in the XCD's L2, a sequence's ranges merged by
+# slices from n_rep ranges on (the long sequence of the first case, most of 32) and by the last
+# arrival below (its second, two or three; its third, one; its fourth has no key at all)
+SHARED = [
+    (32, 8, 0, [6000, 800, 7, 0, 0, 300, 90, 1, 33], [1600, 100, 9, 0, 64, 40, 1, 2, 500]),
+    (8, 8, 0, [11 * i for i in range(20)], [1100 if i in (0, 7, 19) else 3 * i for i in range(20)]),
+    (28, 4, 16, [100 * (i % 7) for i in range(32)] + [3000], [400 - 12 * i for i in range(33)]),   # a pair per two CUs
+    (4, 1, 16, [15000 * (i % 30 == 7) + 5 * i for i in range(64)], [10 + i for i in range(64)]),   # one kv head
+]
+
+
+@pytest.mark.parametrize("hq,hkv,sink,mids,recents", SHARED)
+def test_ranges_shared_by_length(hq, hkv, sink, mids, recents):
+    """Ragged batches whose ranges are shared out by length, against the oracle, twice on one
+    workspace (the hand-off words come back to rest), then with the device-scope hand-off."""
+    from heterokv import ops
+    print("case: shared ranges %d/%d B=%d" % (hq, hkv, len(mids)), flush=True)
+    c = Case(500 + len(mids), len(mids), hq, hkv, sink, mids, recents)
+    assert _shared_ranges(c) > len(mids)
+    for ws in (ops.DecodeWorkspace(DEV), ops.DecodeWorkspace(DEV, agent_handoff=True)):
+        _check(c, workspace=ws)
+        assert ws.error_flag() == 0
+
+
+@pytest.mark.parametrize("hq,hkv,sink,mids,recents", SHARED[:1] + SHARED[3:])
+def test_shared_ranges_with_scores(hq, hkv, sink, mids, recents):
+    """Score outputs of a launch with shared-out ranges (both schedules and hand-offs) against
+    one with three ranges for every sequence: the scores bit for bit (one product each), the
+    softmax max too, the sum up to its order; items past a length untouched."""
+    from heterokv import ops
+    print("case: shared ranges with scores %d/%d" % (hq, hkv), flush=True)
+    c = Case(600 + len(mids), len(mids), hq, hkv, sink, mids, recents)
+    assert _shared_ranges(c) > 0
+    n = sum(mx for _, _, mx in c.zones) + c.maxmid
+
+    def run(splits, det, ws):
+        scores = torch.full((c.B, hq, n), 7.0, dtype=torch.float32, device=DEV)
+        stats = torch.zeros((c.B, hq, 2), dtype=torch.float32, device=DEV)
+        out = ops.decode_attention(c.q.to(DEV), zones=c.zones, pool=c.pool, block_table=c.bt.to(DEV),
+                                   int4_lens=c.int4_lens.to(DEV), int4_max_len=c.maxmid, splits=splits,
+                                   deterministic=det, scores=scores, score_stats=stats, workspace=ws)
+        assert ws.error_flag() == 0
+        return scores.cpu(), stats.cpu(), out.float().cpu()
+
+    want = run(3, True, ops.DecodeWorkspace(DEV))
+    for det in (True, False):
+        for agent in (False, True):
+            got = run(0, det, ops.DecodeWorkspace(DEV, agent_handoff=agent))
+            assert torch.equal(got[0], want[0])
+            assert torch.equal(got[1][..., 0], want[1][..., 0])
+            # sums of up to 2^14 float32 terms in another order
+            assert torch.allclose(got[1][..., 1], want[1][..., 1], rtol=2.0 ** -23 * 128, atol=0)
+            assert (got[2] - want[2]).abs().max().item() <= TOL
