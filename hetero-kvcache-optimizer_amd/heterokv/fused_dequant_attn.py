@@ -18,7 +18,9 @@ value, a decode placement failure) go to a per-device error word that is read wi
 blocking at the next call -- a later call raises HeteroKVError -- or at once by
 check_errors().
 """
+import collections
 import math
+import threading
 from typing import Optional
 
 import torch
@@ -28,16 +30,51 @@ from ._lib import HeteroKVError
 
 
 _ERR = {}   # device -> ErrorWord shared by the calls on that device
-_WS = {}    # device -> DecodeWorkspace shared by the decode calls on that device
+_WS = collections.OrderedDict()   # (device, raw stream) -> DecodeWorkspace, the last used at the end
+_WS_LIMIT = 32   # the oldest goes beyond that (its memory returns to its own stream's allocator pool)
+_AGENT = set()   # devices on which a launch's ranges did not share an XCD: device-scope hand-off
+_LOCK = threading.Lock()
 
 
 def _errword(device):
-    w = _ERR.get(device)
-    if w is None:
-        w = _ERR[device] = ops.ErrorWord(device)
-        _WS[device] = ops.DecodeWorkspace(device)
-        w.on_error = lambda bits: _WS[device].placement_failed() if bits & _lib.ERR_BIT_PLACEMENT else None
+    with _LOCK:
+        w = _ERR.get(device)
+        if w is None:
+            w = _ERR[device] = ops.ErrorWord(device)
+            w.on_error = lambda bits: _placement_failed(device) if bits & _lib.ERR_BIT_PLACEMENT else None
     return w
+
+
+def _workspace(device, stream):
+    """The decode workspace of calls on `device` in `stream` (a raw stream): launches that share
+    one are ordered by their stream, so every stream has its own."""
+    key = (device, stream)
+    with _LOCK:
+        ws = _WS.get(key)
+        if ws is None:
+            ws = _WS[key] = ops.DecodeWorkspace(device, agent_handoff=device in _AGENT)
+            while len(_WS) > _WS_LIMIT:
+                _WS.popitem(last=False)
+        else:
+            _WS.move_to_end(key)
+    return ws
+
+
+def _call_workspace(device):
+    """This call's workspace.  Under graph capture one of its own: the fill that clears it is
+    then part of every replay, and no other call or graph shares it."""
+    if torch.cuda.is_current_stream_capturing():
+        return ops.DecodeWorkspace(device, agent_handoff=device in _AGENT)
+    return _workspace(device, ops.stream_ptr(device).value)
+
+
+def _placement_failed(device):
+    """Tickets of this device's workspaces may be left inconsistent: none is used again (a new
+    one is cleared in its own stream), and all launches use the device-scope hand-off."""
+    with _LOCK:
+        _AGENT.add(device)
+        for key in [k for k in _WS if k[0] == device]:
+            del _WS[key]
 
 
 def check_errors(device=None) -> None:
@@ -83,7 +120,8 @@ def fused_dequant_attn_decode(q: torch.Tensor, k_data: torch.Tensor, k_scales: t
     err = _errword(q.device)
     err.poll()
     qq = _as_kernel_q(q, err)
-    out = ops.fused_decode(qq, kd, vd, k_scales, v_scales, k_zps, v_zps, sm_scale, _WS[q.device], err, qq.dtype)
+    out = ops.fused_decode(qq, kd, vd, k_scales, v_scales, k_zps, v_zps, sm_scale,
+                           _call_workspace(q.device), err, qq.dtype)
     err.post()
     return out.to(q.dtype)
 

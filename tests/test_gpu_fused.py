@@ -102,3 +102,27 @@ def test_fused_forward_row_rule(hq, hkv, S, Sq, monkeypatch):
     print("case: fused forward rows %d" % (hq // hkv * Sq), flush=True)
     x = _inputs(11, 2, hq, hkv, S, Sq, torch.float16)
     _check(fused_dequant_attn_forward(x[0].to(DEV), *[_dev(t) for t in x[1:]]), _reference(*x), torch.float16)
+
+
+def test_fused_decode_on_two_streams():
+    """Overlapping calls on two streams, neither ordered after the other: every result against
+    the oracle (with one workspace they would mix their partial states)."""
+    from heterokv import fused_dequant_attn as fda
+    print("case: fused decode on two streams", flush=True)
+    xs = [_inputs(21 + i, 1, 8, 8, 3000 + 500 * i, 1, torch.float16) for i in range(2)]
+    args = [(x[0].to(DEV),) + tuple(_dev(t) for t in x[1:]) for x in xs]
+    refs = [_reference(*x) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(DEV) for _ in range(2)]
+    outs = [[], []]
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs[i].append(fda.fused_dequant_attn_decode(*args[i]))
+    torch.cuda.synchronize()
+    keys = {(torch.device(DEV), s.cuda_stream) for s in streams}
+    assert keys <= set(fda._WS) and len({id(fda._WS[k]) for k in keys}) == 2
+    for i in range(2):
+        for o in outs[i]:
+            _check(o, refs[i], torch.float16)
+    fda.check_errors(DEV)

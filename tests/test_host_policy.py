@@ -160,3 +160,32 @@ def test_decode_range_plan(B, hq, hkv, mid, zones, own, want):
     if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("a device of another CU count")
     assert ops.decode_ranges(B, hq, hkv, mid, zones, own_lens=own) == want
+
+
+def test_fused_decode_workspace_per_stream(monkeypatch):
+    """Every (device, stream) has a workspace of its own, made once also by several threads; the
+    number kept is bounded; a placement failure drops the device's and switches the hand-off."""
+    import threading
+    import torch
+    from heterokv import fused_dequant_attn as fda
+    monkeypatch.setattr(fda, "_WS", type(fda._WS)())
+    monkeypatch.setattr(fda, "_AGENT", set())
+    d0, d1 = torch.device("cuda:0"), torch.device("cuda:1")   # nothing is allocated before get()
+    a = fda._workspace(d0, None)
+    got = []
+    threads = [threading.Thread(target=lambda: got.append(fda._workspace(d0, 16))) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len({id(w) for w in got}) == 1 and got[0] is not a
+    other = fda._workspace(d1, None)
+    assert fda._workspace(d0, None) is a and other is not a
+    for i in range(fda._WS_LIMIT - 1):
+        fda._workspace(d0, 1000 + i)
+    assert len(fda._WS) == fda._WS_LIMIT
+    assert fda._workspace(d0, None) is a                # used last of the first three: still kept
+    assert fda._workspace(d1, None) is not other        # the oldest went
+    fda._placement_failed(d0)
+    b = fda._workspace(d0, None)
+    assert b is not a and b.agent_handoff and not fda._workspace(d1, None).agent_handoff
