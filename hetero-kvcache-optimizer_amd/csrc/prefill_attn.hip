@@ -109,8 +109,9 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     const int T = (t1 - t0 + kFlatBufs - 1) / kFlatBufs * kFlatBufs;
     // of these, a wave attends those up to its last query's
     int Tc = row0 < p.Sq * p.nrep ? T : 0;
+    const int q_hi = min((row0 + kPfQ - 1) / p.nrep, p.Sq - 1);
     if (kKind == kKindF16 && tm.nc > 0 && Tc > 0) {
-        const int last = tm.nf() - tm.nc + min((row0 + kPfQ - 1) / p.nrep, p.Sq - 1) / kPfT;
+        const int last = tm.nf() - tm.nc + q_hi / kPfT;
         Tc = min(T, max(0, last - t0 + kFlatBufs) / kFlatBufs * kFlatBufs);
     }
 
@@ -125,7 +126,10 @@ __device__ __forceinline__ void attend(const PrefillParams& p, int wg, uint8_t* 
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
-    const FlatWave fw{b, h, wt, lane, n, hh, qrow, row0 / p.nrep};
+    if (kKind == kKindF16) {   // read behind the loop's first barrier
+        for (int i = threadIdx.x; i < kZeroBytes / 16; i += kFlatThreads) ((pu4*)(lds + kFlatLdsBytes))[i] = pu4{0u, 0u, 0u, 0u};
+    }
+    const FlatWave fw{b, h, wt, lane, n, hh, qrow, row0 / p.nrep, q_hi};
     if (T > 0) {
         if (team == 0) {
             Stage<kKind, 0> pol(p, tm, fw, t0, t1);
@@ -340,9 +344,10 @@ int launch_slice(PrefillParams& p, const Plan& pl, bool ref, hipStream_t stream)
             if (p.pieces[k] > 0) kinds |= 1 << k;
         }
         if (ref) kinds = 1 << (p.int4_max_len % 4 == 0 ? kKindRefVec : kKindRef);
-        HKV_RAISE_LDS(fns[kinds], kFlatLdsBytes, raised[kinds]);
-        hipLaunchKernelGGL(fns[kinds], dim3(all * (unsigned)(p.pieces[0] + p.pieces[1])), dim3(kFlatThreads),
-                           kFlatLdsBytes, stream, p);
+        const int lds = kFlatLdsBytes + (kinds & (1 << kKindF16) ? kZeroBytes : 0);
+        HKV_RAISE_LDS(fns[kinds], lds, raised[kinds]);
+        hipLaunchKernelGGL(fns[kinds], dim3(all * (unsigned)(p.pieces[0] + p.pieces[1])), dim3(kFlatThreads), lds, stream,
+                           p);
         HKV_LAUNCH_CHECK("prefill_attn_kernel");
     }
     if (pl.finish == kFinishPieces) {

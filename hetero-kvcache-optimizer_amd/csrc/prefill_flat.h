@@ -41,6 +41,9 @@ constexpr int kVOff = kPfT * kKRow;
 constexpr int kDataBytes = kVOff + kHeadDim * kVRow;
 constexpr int kFacBytes = kPfT * 4;
 constexpr int kFlatLdsBytes = kFlatBufs * (kFacBytes + kDataBytes);
+// Behind the buffers, in kernels with fp16 tiles: V^T rows of zeros (F16Stage::values).
+constexpr int kZeroBytes = kHeadDim * kVRow;
+static_assert(kFlatLdsBytes + kZeroBytes <= 160 * 1024, "one workgroup's LDS");
 
 __device__ __forceinline__ uint8_t* flat_buf(uint8_t* lds, int i) { return lds + kFlatBufs * kFacBytes + i * kDataBytes; }
 __device__ __forceinline__ uint8_t* flat_bias(uint8_t* lds, int i) { return lds + i * kFacBytes; }
@@ -66,9 +69,9 @@ __device__ __forceinline__ void flat_barrier() {
 }
 
 // A wave's place: staging share wt (of 4) and lane; its lane's query (row / n_rep) and the
-// wave's lowest one.
+// wave's lowest and highest ones.
 struct FlatWave {
-    int b, h, wt, lane, n, hh, qrow, q_lo;
+    int b, h, wt, lane, n, hh, qrow, q_lo, q_hi;
 };
 
 // QK: S^T[64 tok x 32 q] = K . Q^T + c0.  The two token blocks' accumulators are two
@@ -185,6 +188,8 @@ __device__ __forceinline__ void pv_flat(const uint8_t* vt, int n, int hh, const 
 //   tvalid(x)                  valid tokens of tile x (0 for an empty tile)
 //   mask(x, S)                 extra per-score masking of tile x (chunk tiles that reach
 //                              past a query), a wave-uniform branch
+//   values(x, buf, lds)        the buffer whose V^T rows tile x's probabilities weigh: buf, or
+//                              zeros for a tile that no query of the wave sees (fp16)
 // and (m, l, acc) carry the online softmax of this wave's rows in and out.
 template <class Pol>
 __device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const FlatWave& w, uint8_t* lds, const ph8 (&qf)[8],
@@ -247,7 +252,7 @@ __device__ __forceinline__ void flat_tiles(Pol& pol, const TileMap& tm, const Fl
             }
             __builtin_amdgcn_sched_barrier(0);
             // B: PV(t) beside the staging of tile t+2 and the row sum
-            pv_flat(bt, w.n, w.hh, P, acc);
+            pv_flat(pol.values(t, bt, lds), w.n, w.hh, P, acc);
             pol.stage(uu % Pol::kRing, flat_buf(lds, (uu + 2) % kFlatBufs), flat_bias(lds, (uu + 2) % kFlatBufs), t + 2);
             sm_sum(P, l);
             asm volatile("" ::"v"(l));   // keep the row sum beside this tile's MFMAs

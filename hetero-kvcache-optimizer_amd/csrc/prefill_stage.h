@@ -171,6 +171,7 @@ struct Int4Stage {
         }
     }
     __device__ void mask(int, pf16v (&)[2]) const {}
+    __device__ const uint8_t* values(int, const uint8_t* buf, uint8_t*) const { return buf; }
 };
 
 // The fp16 staging policy of the tile loop: one register slot per wave (64 bytes per
@@ -185,6 +186,7 @@ struct F16Stage {
     const PrefillParams& p;
     const FlatWave& w;
     const int chunk0;      // the loop's tile of the chunk's first tokens (past every tile without a chunk)
+    const int last;        // the last tile that a query of the wave sees (past every tile without a chunk)
     int tiles;             // tiles not yet loaded
     int si, left, len;     // the source, its tiles not yet loaded, its tokens from the next tile on
     const uint16_t* base;  // the next tile's K rows (team 0) or V tiles (team 1)
@@ -192,7 +194,8 @@ struct F16Stage {
     u4 slot[4];
 
     __device__ F16Stage(const PrefillParams& p_, const TileMap& tm, const FlatWave& w_, int x0, int x1)
-        : p(p_), w(w_), chunk0(tm.nc > 0 ? tm.nz_t[0] + tm.nz_t[1] + tm.nz_t[2] - x0 : 1 << 24), tiles(x1 - x0) {
+        : p(p_), w(w_), chunk0(tm.nc > 0 ? tm.nz_t[0] + tm.nz_t[1] + tm.nz_t[2] - x0 : 1 << 24),
+          last(chunk0 + w_.q_hi / kPfT), tiles(x1 - x0) {
         si = 0;
         int x = x0;
 #pragma unroll
@@ -283,6 +286,13 @@ struct F16Stage {
                 for (int r = 0; r < 16; ++r)
                     if (tb * 32 + 8 * (r >> 2) + 4 * w.hh + (r & 3) > lim) S[tb][r] = -INFINITY;
         }
+    }
+    // Past the wave's last query the probabilities are zeros, but the loop's rounds go on for up
+    // to three tiles: a non-finite value of a token there would turn the wave's outputs to NaN
+    // (0 x inf), so these tiles weigh zeros.  Within the last tile it does, as in any product
+    // with masked probabilities.
+    __device__ const uint8_t* values(int x, const uint8_t* buf, uint8_t* lds) const {
+        return x > last ? lds + kFlatLdsBytes - kVOff : buf;
     }
 };
 
@@ -398,6 +408,7 @@ struct RefStage {
         }
     }
     __device__ void mask(int, pf16v (&)[2]) const {}
+    __device__ const uint8_t* values(int, const uint8_t* buf, uint8_t*) const { return buf; }
 };
 
 }  // namespace hkv

@@ -297,6 +297,42 @@ def test_paired_half_units(hq, hkv, sq, recent):
     _case(80 + sq, 1, hq, hkv, sq, 0, [0], [recent])
 
 
+@pytest.mark.parametrize("hq,hkv,mid,rec", [(2, 2, 0, 0), (8, 2, 0, 70), (16, 2, 700, 30), (14, 2, 0, 10), (32, 8, 9000, 64)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_nonfinite_values_of_later_tokens(hq, hkv, mid, rec, value):
+    """A non-finite V of a chunk token, whose probability is zero for the queries before it, stays
+    out of the outputs of every query whose wave of 32 rows ends in an earlier 64-token tile (a
+    wave's tiles go in rounds of four, one past them weighs zeros): the same bits as without it."""
+    from heterokv import ops
+    print("case: non-finite V %d/%d mid %d rec %d %s" % (hq, hkv, mid, rec, value), flush=True)
+    sq, bad = 450, 137
+    g = torch.Generator().manual_seed(91)
+    mk = lambda n, h: torch.randn((1, h, n, 128), generator=g).half().to(DEV)   # noqa: E731
+    kw = {"chunk_k": mk(sq, hkv), "chunk_v": mk(sq, hkv)}
+    if mid:
+        pool = ops.Int4Pool((mid + 15) // 16, hkv, DEV)
+        bt = torch.arange((mid + 15) // 16, dtype=torch.int32, device=DEV)[None]
+        ops.pack_tokens(pool, mk(mid, hkv), mk(mid, hkv), 0, bt)
+        kw.update(pool=pool, block_table=bt, int4_max_len=mid)
+    if rec:
+        z = ops.F16Zone(1, hkv, rec, DEV)
+        z.write(mk(rec, hkv), mk(rec, hkv), 0)
+        kw["zones"] = [(z, None, rec)]
+    q = mk(sq, hq)
+    from heterokv._lib import load
+    ws = torch.empty(load().hkv_prefill_workspace_bytes(1, hq, sq), dtype=torch.uint8, device=DEV)
+    nrep = hq // hkv
+    # a wave's 32 rows: with n_rep no divisor of 32 they may begin in one tile and end in the next
+    safe = 128 if 32 % nrep == 0 else 128 - 31 // nrep - 1
+    for w in (None, ws):   # with room for pieces, and without
+        kw["chunk_v"][:, :, bad] = 0.5
+        want = ops.prefill_attention(q, workspace=w, **kw)
+        kw["chunk_v"][:, :, bad] = value
+        got = ops.prefill_attention(q, workspace=w, **kw)
+        assert torch.equal(got[:, :, :safe], want[:, :, :safe])
+        assert torch.isfinite(want).all() and not torch.isfinite(got[:, :, bad:]).any()
+
+
 def test_more_pairs_than_one_grid_holds():
     """65535 sequences of 129 heads with one query each: more workgroups of 512 threads than one
     grid takes (2^32 threads), so the sequences go in two launches.  Sequence b repeats sequence
