@@ -639,26 +639,33 @@ def fused_decode(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale
     return out
 
 
-# Query rows per kv head, and query-token products of the call, from which fused_forward repacks
-# the codes: a tile of unpacked codes takes the prefill kernel longer, once per 256 rows, and
-# repacking costs one pass over the codes and some launches.  What each route takes above the
-# prefill kernel on repacked records alone (both include the error word's copy), direct and
-# repacked, in us: 32/8 heads, 1024 queries over 1024 tokens 0.6 and 7.4, over 16001 (5.2e8
-# products) 12.1 and 8.2; 2048 queries over 6260 (4.1e8) 3.4 and 8.7, over 16001 (1.0e9) 33 and
-# 8.0; 28/4 heads, 1024 queries over 6260 (1.8e8) 9.5 and 12.9; four sequences of 32/8 heads,
-# 1765 queries over 1024 (2.3e8) 11.0 and 8.3, over 6260 (1.4e9) 38 and 3.8.
-_REPACK_ROWS = 3072
-_REPACK_WORK = 1 << 28
+# What each route of fused_forward takes above the prefill kernel on a ready pool, in us: a tile of
+# unpacked codes takes longer than a packed one (rows of 4 k tokens, and others), on every round of
+# the CUs; repacking is one pass over the codes and some launches.  Direct and repacked, measured
+# (both with the error word's copy, ~6): 32/8 heads, 2048 queries over 2500 tokens 13 and 18, 6260
+# 21 and 23, 16000 39 and 27, 16001 62 and 27; four sequences of them, 1024 queries over 6260 34
+# and 35, 2048 over 1024 19 and 18, over 6260 72 and 34; 28/4 heads, 2048 over 6260 20 and 18;
+# 32/32 heads, 2048 over 16000 38 and 57, over 16001 69 and 56, two sequences of them 123 and 116,
+# 188 and 109.  Over 140 sizes the choice is at most 7 us off the better route (fixed lines at 3072
+# rows per kv head and 2^28 query-token products: 78).
+_TILE_US, _ODD_TILE_US = 0.15, 0.22
+_REPACK_US, _REPACK_US_PER_TOKEN = 6.0, 0.08 / 1024
+_UNIT_ROWS, _TILE_TOKENS, _CUS = 256, 64, 256   # the prefill kernel's; workgroups of one round
 
 
 def _repacks(batch, q_heads, kv_heads, queries, tokens):
-    rows = queries * (q_heads // kv_heads) if kv_heads else 0
-    return rows >= _REPACK_ROWS and batch * q_heads * queries * tokens >= _REPACK_WORK
+    if kv_heads <= 0:
+        return False
+    rounds = batch * kv_heads * -(-queries * (q_heads // kv_heads) // _UNIT_ROWS) / _CUS
+    if rounds > 1:
+        rounds = math.ceil(rounds)   # a part of a round: the keys of its units are split
+    direct = (_ODD_TILE_US if tokens % 4 else _TILE_US) * -(-tokens // _TILE_TOKENS) * rounds
+    return direct > _REPACK_US + _REPACK_US_PER_TOKEN * batch * kv_heads * tokens
 
 
 def fused_forward(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps, sm_scale, err, out_dtype):
-    """Attention of q [B, Hq, Sq, 128] over every unpacked token: hkv_fused_forward, or with
-    many query rows and tokens hkv_repack_codes and hkv_prefill_attn."""
+    """Attention of q [B, Hq, Sq, 128] over every unpacked token: hkv_fused_forward, or where the
+    codes are read often (_repacks) hkv_repack_codes and hkv_prefill_attn."""
     _check_fused(q, k_codes, v_codes, k_scales, v_scales, k_zps, v_zps)
     B, H, T, _ = k_codes.shape
     if _repacks(B, q.shape[1], H, q.shape[2], T):

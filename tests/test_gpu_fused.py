@@ -94,10 +94,10 @@ def test_fused_forward_split_keys(hkv, S, Sq):
 
 @pytest.mark.parametrize("hq,hkv,S,Sq", [(12, 1, 70, 255), (12, 1, 70, 256), (12, 1, 33, 257)])
 def test_fused_forward_row_rule(hq, hkv, S, Sq, monkeypatch):
-    """Query rows per kv head on both sides of the line at which the codes are repacked (into a
-    pool whose last block is written only in part), without the line on the call's work."""
+    """Query rows per kv head around 3072, those from there on with the codes repacked (into a
+    pool whose last block is written only in part), as calls with many more keys have it."""
     from heterokv import fused_dequant_attn_forward, ops
-    monkeypatch.setattr(ops, "_REPACK_WORK", 0)
+    monkeypatch.setattr(ops, "_repacks", lambda b, qh, kh, queries, tokens: queries * qh >= 3072 * kh)
     assert ops._repacks(2, hq, hkv, Sq, S) == (Sq >= 256)
     print("case: fused forward rows %d" % (hq // hkv * Sq), flush=True)
     x = _inputs(11, 2, hq, hkv, S, Sq, torch.float16)

@@ -119,20 +119,18 @@ def test_window_selection_follows_score_changes():
     assert m._top_chunks(0, keys, 2) == ("l0_e0", "l0_e5")
 
 
-@pytest.mark.parametrize("rows", [1, 1 << 30])
-def test_fused_forward_refuses_another_batch_on_both_routes(monkeypatch, rows):
+@pytest.mark.parametrize("repack", [True, False])
+def test_fused_forward_refuses_another_batch_on_both_routes(monkeypatch, repack):
     """Queries of more sequences than the codes are refused before either route (the block
     table made for the codes has no row for them): no pool is made, no kernel is reached."""
     from heterokv import HeteroKVError, ops
     reached = []
     monkeypatch.setattr(ops, "_require_gpu", lambda *ts: None)
-    monkeypatch.setattr(ops, "_REPACK_ROWS", rows)
-    monkeypatch.setattr(ops, "_REPACK_WORK", 0)
+    monkeypatch.setattr(ops, "_repacks", lambda *a: repack)
     for name in ("Int4Pool", "repack_codes", "prefill_attention", "load"):
         monkeypatch.setattr(ops, name, lambda *a, _n=name, **k: reached.append(_n))
     q = torch.zeros((2, 4, 8, 128), dtype=torch.float16)
     codes, rows_ = torch.zeros((1, 2, 32, 128), dtype=torch.uint8), torch.zeros((1, 2, 32))
-    assert ops._repacks(2, 4, 2, 8, 32) == (rows == 1)
     with pytest.raises(HeteroKVError, match="q must be"):
         ops.fused_forward(q, codes, codes, rows_, rows_, rows_, rows_, 1.0, SimpleNamespace(dev=None, ptr=lambda: 0),
                           torch.float16)
@@ -189,3 +187,15 @@ def test_fused_decode_workspace_per_stream(monkeypatch):
     fda._placement_failed(d0)
     b = fda._workspace(d0, None)
     assert b is not a and b.agent_handoff and not fda._workspace(d1, None).agent_handoff
+
+
+@pytest.mark.parametrize("B,hq,hkv,Sq,T,repack", [
+    # sizes at which one route measured clearly faster
+    (1, 32, 8, 2048, 2500, False), (1, 32, 8, 2048, 16000, True), (1, 32, 8, 2048, 16001, True),
+    (4, 32, 8, 512, 6260, False), (4, 32, 8, 2048, 6260, True), (1, 32, 32, 2048, 16000, False),
+    (1, 32, 32, 2048, 16001, True), (2, 32, 32, 2048, 16001, True), (2, 32, 32, 1024, 16000, False),
+    (4, 28, 4, 1024, 6260, True), (1, 32, 8, 512, 16000, False), (1, 32, 32, 512, 4096, False),
+])
+def test_fused_forward_route(B, hq, hkv, Sq, T, repack):
+    from heterokv import ops
+    assert ops._repacks(B, hq, hkv, Sq, T) == repack
