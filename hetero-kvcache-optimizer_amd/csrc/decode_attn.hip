@@ -74,7 +74,8 @@ constexpr int kPrefetch = HKV_DECODE_PREFETCH;  // INT4 block pairs in flight pe
 #define HKV_DECODE_F16_DEPTH 1
 #endif
 constexpr int kF16Depth = HKV_DECODE_F16_DEPTH;
-constexpr int kMaxSplits = 64;           // the slice merge takes 16 x 4 states
+constexpr int kMaxSplits = 64;           // the slice merge takes 16 x 4 states, or
+constexpr int kL2Ranges = 32;            // 4 x 8: the most with the XCD-local hand-off (32 CUs)
 constexpr int kLineWords = 64;           // ints per 256-byte hand-off line
 // Slice merge: the pair's arrival word holds the arrivals of the current launch in bits
 // 0-15, a generation in bits 16-29 that the last arrival advances (clearing the count),
@@ -1308,7 +1309,9 @@ __global__ __launch_bounds__(kThreads) void decode_attn_kernel(typename KernelPa
             (void*)parts, 0, (int)(nsplit * sstride * sizeof(float)), 0x00020000);
         const int S = slice_outputs;
         const int sl0 = slices == 2 ? 0 : split, sl1 = slices == 2 ? nsplit : split + 1;
-        const int lsh = nsplit > 32 ? 4 : 2;
+        // (an XCD-local pair has no more than 32 resident ranges, one per CU of its XCD; with the
+        // 16-lane code in its kernel too, eight layers at 32K took 135.6 us, without 133.7)
+        const int lsh = !kL2 && nsplit > kL2Ranges ? 4 : 2;
         for (int sl = sl0; sl < sl1; ++sl) {
             for (int t = threadIdx.x; t < S << lsh; t += kThreads) {
                 const int o = sl * S + (t >> lsh), q = t & ((1 << lsh) - 1);
@@ -1774,7 +1777,7 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
     p.nxcc = num_xcc();
     // one range per pair needs no hand-off (and must not leave a mask bit behind)
     // (shared-out ranges: the kv heads are innermost in the workgroup ids, not the pairs)
-    p.xcc_local = ((lin > 0 ? a->num_kv_heads : BH) % p.nxcc) == 0 && (ms > 1 || lin > 0) &&
+    p.xcc_local = ((lin > 0 ? a->num_kv_heads : BH) % p.nxcc) == 0 && (ms > 1 || lin > 0) && lin <= kL2Ranges &&
                           !(a->flags & HKV_DECODE_AGENT_HANDOFF)
                       ? 1
                       : 0;
@@ -1794,7 +1797,8 @@ static int decode_launch(const HkvDecodeArgs* a, void* wsp, size_t ws_bytes, voi
         const int S = (nout + ms - 1) / ms;
         // Shared-out ranges decide per pair in the kernel.
         p.slice_outputs = S;
-        p.coop = (ms > 1 && (int64_t)BH * ms <= num_cus() && S <= 128 && ms < kArrivedMask) ? 1 : 0;
+        p.coop = (ms > 1 && (int64_t)BH * ms <= num_cus() && S <= 128 && ms < kArrivedMask &&
+                  (ms <= kL2Ranges || !p.xcc_local)) ? 1 : 0;
         const char* mw = getenv("HKV_DECODE_MERGE_WAIT_TICKS");
         p.merge_wait = (mw && mw[0]) ? strtoull(mw, nullptr, 10) : kMergeWaitTicks;
     }
