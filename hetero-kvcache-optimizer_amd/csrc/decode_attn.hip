@@ -1483,7 +1483,9 @@ int num_cus() {
 // ranges 28.8 us).  Within that, a range holds at least two units (an fp16 tile or a pair of
 // INT4 blocks), since a short range costs little and the slice merge needs at least n_rep
 // ranges (507 tokens of 32/8 heads: 3 ranges of ~96 KB 8.8 us, 16 ranges 6.9 us, 32 ranges
-// 7.1 us; 28/4 heads 12.4, 8.4 and 8.4 us).  Few units stay in one range, without a
+// 7.1 us; 28/4 heads 12.4, 8.4 and 8.4 us; at most 5% off the best count over 60 sizes of one
+// sequence, the most at 162 INT4 beside 2832 fp16 tokens of 32/8 heads: 32 ranges 11.9 us, 16
+// 11.3; of 5000 beside 300 they take 11.7 and 12.2).  Few units stay in one range, without a
 // hand-off: up to kOneRange, two per wave (164 tokens: 5.9 us against 6.8 us), and with the
 // dearer last-arrival merge of fewer than n_rep ranges while s ranges take no more than
 // kOneRangeWide units off one (units (s - 1) / s; pairs for two ranges each, n_rep 4 to 8: 36

@@ -27,7 +27,8 @@
 //   kFinishSerial   both kinds, one piece each: the fp16 kernel runs first, the INT4 kernel
 //                   merges its states into its own and writes the output
 // A workgroup takes one piece: with a loop over several, the tile loop's register
-// allocation (248 of 256) no longer holds.
+// allocation no longer holds (248 of 256 for INT4 tiles; all 256 for the other kinds, which
+// spill 2 to 11, only kKindRefVec's loop reloading four of them).
 #pragma once
 
 #include "hkv_internal.h"

@@ -11,9 +11,10 @@ exactly that formula, and it also accepts GQA (q heads a multiple of kv heads).
 
 The reference passes unpacked codes (one uint8 per value) with per-token
 scales/zps [B, H, S], which the kernels attend as they are: the split-K decode kernel
-(hkv_fused_decode) and the MFMA prefill kernel (hkv_fused_forward; with many query rows per
-kv head the codes are repacked into block records first, which the rows then share).  q may be fp16 or bf16 (bf16 is narrowed to
-fp16 operands exactly within the fp16 range).  Device errors (an out-of-range bf16
+(hkv_fused_decode) and the MFMA prefill kernel (hkv_fused_forward; where the query rows read
+the codes often, they are repacked into block records first).  Calls may run on several streams
+at once.  q may be fp16 or bf16 (bf16 is narrowed to fp16 operands exactly within the fp16
+range).  Device errors (an out-of-range bf16
 value, a decode placement failure) go to a per-device error word that is read without
 blocking at the next call -- a later call raises HeteroKVError -- or at once by
 check_errors().
