@@ -424,16 +424,27 @@ SHARED = [
 
 
 @pytest.mark.parametrize("hq,hkv,sink,mids,recents", SHARED)
-def test_ranges_shared_by_length(hq, hkv, sink, mids, recents):
-    """Ragged batches whose ranges are shared out by length, against the oracle, twice on one
-    workspace (the hand-off words come back to rest), then with the device-scope hand-off."""
+def test_ranges_shared_by_length(hq, hkv, sink, mids, recents, monkeypatch):
+    """Ragged batches whose ranges are shared out by length, against the oracle, in both
+    schedules and with both hand-offs, several times on one workspace (the hand-off words come
+    back to rest), also with ranges that stop waiting at once for the others."""
     from heterokv import ops
     print("case: shared ranges %d/%d B=%d" % (hq, hkv, len(mids)), flush=True)
     c = Case(500 + len(mids), len(mids), hq, hkv, sink, mids, recents)
     assert _shared_ranges(c) > len(mids)
+    ref = c.oracle()
     for ws in (ops.DecodeWorkspace(DEV), ops.DecodeWorkspace(DEV, agent_handoff=True)):
-        _check(c, workspace=ws)
-        assert ws.error_flag() == 0
+        for wait in (None, "0", "0", None):
+            if wait is None:
+                monkeypatch.delenv("HKV_DECODE_MERGE_WAIT_TICKS", raising=False)
+            else:
+                monkeypatch.setenv("HKV_DECODE_MERGE_WAIT_TICKS", wait)
+            for det in (False, True):
+                got = c.run(workspace=ws, deterministic=det)
+                err = np.abs(got - ref).max()
+                print("  wait=%s deterministic=%s max abs err %.3e" % (wait, det, err), flush=True)
+                assert np.all(np.isfinite(got)) and err <= TOL
+                assert ws.error_flag() == 0
 
 
 @pytest.mark.parametrize("hq,hkv,sink,mids,recents", SHARED[:1] + SHARED[3:])
