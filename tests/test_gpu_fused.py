@@ -126,3 +126,29 @@ def test_fused_decode_on_two_streams():
         for o in outs[i]:
             _check(o, refs[i], torch.float16)
     fda.check_errors(DEV)
+
+
+def test_fused_decode_captured_call():
+    """A captured call's replays, with new queries and with eager calls on other streams between
+    them (the graph clears and owns its workspace), against the oracle."""
+    from heterokv import fused_dequant_attn as fda
+    print("case: fused decode in a graph", flush=True)
+    x = _inputs(31, 1, 8, 8, 2500, 1, torch.float16)
+    q = x[0].to(DEV)
+    args = tuple(_dev(t) for t in x[1:])
+    fda.fused_dequant_attn_decode(q, *args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fda.fused_dequant_attn_decode(q, *args)
+    side = torch.cuda.Stream(DEV)
+    for scale in (1.0, -0.5, 2.0, 0.25):
+        q.copy_(x[0] * scale)
+        ref = _reference(x[0] * scale, *x[1:])
+        torch.cuda.synchronize()
+        graph.replay()
+        with torch.cuda.stream(side):
+            eager = fda.fused_dequant_attn_decode(q, *args)
+        torch.cuda.synchronize()
+        _check(out, ref, torch.float16)
+        _check(eager, ref, torch.float16)
